@@ -8,8 +8,8 @@
 //                    owned by 8 lanes of one wave, so passes along rows are
 //                    separated by wave barriers, everything else by
 //                    work-group barriers (nine per position).
-//   k_gather         one work group per 4 x 64 object tile: float64 sums of
-//                    the staged patches in batch order (deterministic).
+//   k_scatter        one work group per object tile: float64 sums of the
+//                    staged patches in batch order (pty_scatter.inc).
 //   k_object_update  normalised object step.
 //   k_probe_partial / k_probe_update   probe step from staged terms.
 //   k_constraint_*   per-iteration object constraints; k_probe_com probe
@@ -493,14 +493,24 @@ struct GatherGpuRunner {
   __device__ __forceinline__ void barrier() { __syncthreads(); }
 };
 
-__device__ __forceinline__ void gather_body(const GatherArgs& a, int tile) {
-  __shared__ GatherShared sh;
+// one 8 x 64 tile per work group, one thread per two pixels, 64-bit frame
+// offsets: the frames beyond a buffer resource's 2 GiB (scatter_in_range).
+// `ntiles`: tiles of the scatter plan, at least as many as this kernel's
+// `own`; the maxima beyond its own are cleared (|P|^2 sums are not negative).
+__device__ __forceinline__ void gather_body(const GatherArgs& a, int tile, int own, int ntiles, GatherShared& sh) {
   Gather::Regs r;
   GatherGpuRunner run{r, GatherSharedView{&sh}, (int)threadIdx.x};
   gather_tile(run, a, tile);
+  if (a.tilemax && threadIdx.x == 0)
+    for (int t = own + tile; t < ntiles; t += own) a.tilemax[t] = 0.f;
 }
 
-__global__ __launch_bounds__(GATHER_THREADS) void k_gather(GatherArgs a) { gather_body(a, (int)blockIdx.x); }
+__global__ __launch_bounds__(GATHER_THREADS) void k_gather(GatherArgs a, int ntiles) {
+  __shared__ GatherShared sh;
+  gather_body(a, (int)blockIdx.x, (int)gridDim.x, ntiles, sh);
+}
+
+#include "pty_scatter.inc"
 
 __device__ float block_max(float v, float* sh) {
   sh[threadIdx.x] = v;
@@ -685,44 +695,64 @@ struct ProbePartialArgs {
   const float* object_pot = nullptr;  // potential V: the patch is exp(i V)
 };
 
+// Sums over the chunk's slots, in batch order: conj(O) * chi (float32 products
+// rounded separately, float64 sums) and |O|^2 (squares and sums in float64,
+// two fused multiply-adds: no square root and no float32 rounding, which a
+// |O| in float32 would cost).
 __device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, int blk, int chunk) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-  __shared__ int anchor[2 * PROBE_CHUNK];
+  __shared__ int2 anchor[PROBE_CHUNK];
   const int S = a.S;
   const int b0 = chunk * PROBE_CHUNK;
   if (b0 >= a.B) return;  // uniform over the work group
   const int nb = min(a.B - b0, PROBE_CHUNK);
-  // the chunk's rounded patch anchors, once per work group: the loop below
-  // then issues only independent object and chi loads
+  // the object index of the chunk's window origins (window rows and columns
+  // in ascending order, origin S/2 before the patch anchor), once per work
+  // group: the loop below then issues only independent object and chi loads
   for (int t = threadIdx.x; t < nb; t += blockDim.x) {
     int idx = a.order[b0 + t];
     idx = ((unsigned)idx < (unsigned)a.N) ? idx : 0;
-    anchor[2 * t] = wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px);
-    anchor[2 * t + 1] = wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py);
+    anchor[t] = make_int2(wrap1(wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px) - S / 2, a.Px),
+                          wrap1(wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py) - S / 2, a.Py));
   }
   __syncthreads();
   const int pix = blk * blockDim.x + threadIdx.x;
   if (pix >= S * S) return;
-  const int i = pix / S, j = pix % S;
-  const int fi = i < S / 2 ? i : i - S;
-  const int fj = j < S / 2 ? j : j - S;
+  // window coordinates of probe pixel (i, j): corner-centred index ^ S/2
+  const unsigned wi = (unsigned)(pix / S) ^ (unsigned)(S / 2), wj = (unsigned)(pix % S) ^ (unsigned)(S / 2);
+  const unsigned Px = a.Px, Py = a.Py;
   const cf* chi = a.chi + (size_t)b0 * S * S + pix;
   double re = 0.0, im = 0.0, so = 0.0;
-  // anchors in the object and |fi|, |fj| <= S/2 <= Px/2, Py/2: one
-  // conditional wrap per side; offsets fit 32 bits (object < 2^31 elements)
-#pragma unroll 8
-  for (int k = 0; k < nb; ++k) {  // batch order
-    const int x0 = anchor[2 * k], y0 = anchor[2 * k + 1];
-    const unsigned off = (unsigned)(wrap1(x0 + fi, a.Px) * a.Py + wrap1(y0 + fj, a.Py));
-    const cf o = a.object_pot ? expi(elem(a.object_pot, off)) : elem(a.object, off);
-    const float ao = hypot_f(o.x, o.y);
-    so += (double)(ao * ao);
-    const cf g = cconjmul_rn(o, elem(chi, (unsigned)(k * S * S)));
+  const auto object = [&](int k) {
+    const int2 w = anchor[k];
+    unsigned r = (unsigned)w.x + wi, q = (unsigned)w.y + wj;
+    r = umin(r, r - Px);  // origin and window coordinate below Px: one wrap
+    q = umin(q, q - Py);
+    return a.object_pot ? expi(elem(a.object_pot, r * Py + q)) : elem(a.object, r * Py + q);
+  };
+  const auto add = [&](cf o, cf c) {
+    const double x = o.x, y = o.y;
+    so = __builtin_fma(x, x, so);
+    so = __builtin_fma(y, y, so);
+    const cf g = cconjmul_rn(o, c);
     re += (double)g.x;
     im += (double)g.y;
+  };
+  constexpr int U = 8;  // slots loaded ahead of their sums
+  int k = 0;
+  for (; k + U <= nb; k += U) {
+    cf o[U], c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      o[u] = object(k + u);
+      c[u] = elem(chi, (unsigned)(k + u) * (unsigned)(S * S));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) add(o[u], c[u]);
   }
+  for (; k < nb; ++k) add(object(k), elem(chi, (unsigned)k * (unsigned)(S * S)));
   double* p = a.part + ((size_t)chunk * S * S + pix) * 3;
   p[0] = re;
   p[1] = im;
@@ -733,14 +763,16 @@ __global__ __launch_bounds__(256) void k_probe_partial(ProbePartialArgs a) {
   probe_partial_body(a, blockIdx.x, blockIdx.y);
 }
 
-// the scatter of a stage (work groups [0, ntiles)) and its probe partial
+// the scatter of a stage (work groups [0, nscatter)) and its probe partial
 // sums (the rest, pixel block fastest) in one launch: both only read the
 // fused pass's staged terms
-__global__ __launch_bounds__(256) void k_gather_probe(GatherArgs g, ProbePartialArgs pa, int ntiles,
-                                                      int pix_blocks) {
+template <int R>
+__global__ __launch_bounds__(256) void k_scatter_probe(GatherArgs g, ScatterPlan plan, int nscatter,
+                                                       ProbePartialArgs pa, int pix_blocks) {
+  __shared__ ScatterShared<R> sh;
   const int b = (int)blockIdx.x;
-  if (b < ntiles) gather_body(g, b);
-  else probe_partial_body(pa, (b - ntiles) % pix_blocks, (b - ntiles) / pix_blocks);
+  if (b < nscatter) scatter_body<R>(g, plan, b, sh);
+  else probe_partial_body(pa, (b - nscatter) % pix_blocks, (b - nscatter) / pix_blocks);
 }
 
 // per-pixel sum of the chunk partials: PROBE_REDUCE_GROUPS contiguous chunk
@@ -1332,11 +1364,17 @@ int launch_fft(const cf* in, cf* out, int batch, int S, bool inv, int natural, h
   return check_launch("k_fft2");
 }
 
-int num_tiles(int Px, int Py) { return gather_num_tiles(Px, Py); }
-
-int launch_gather(const GatherArgs& a, int Px, int Py, hipStream_t stream) {
-  hipLaunchKernelGGL(k_gather, dim3(num_tiles(Px, Py)), dim3(GATHER_THREADS), 0, stream, a);
-  return check_launch("k_gather");
+int launch_scatter(const GatherArgs& a, hipStream_t stream) {
+  const ScatterPlan plan = scatter_plan(a.Px, a.Py);
+  if (!scatter_in_range(a.B, a.S)) {
+    hipLaunchKernelGGL(k_gather, dim3(gather_num_tiles(a.Px, a.Py)), dim3(GATHER_THREADS), 0, stream, a,
+                       plan.tiles_x * plan.tiles_y);
+    return check_launch("k_gather");
+  }
+  const dim3 grid(scatter_blocks(a.Px, a.Py)), blk(256);
+  if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter<1>, grid, blk, 0, stream, a, plan);
+  else hipLaunchKernelGGL(k_scatter<4>, grid, blk, 0, stream, a, plan);
+  return check_launch("k_scatter");
 }
 
 int grid_for(long long n, int threads, int cap = 4096) {
@@ -1404,6 +1442,23 @@ int launch_probe_apply(cf* probe, double* ws, int S, int B, float step, float nm
   hipLaunchKernelGGL(k_probe_apply, dim3(nblk), dim3(256), 0, stream, probe, gsum, osum, bmax, nblk, npix, step,
                      c1, c2, replace);
   return check_launch("k_probe_apply");
+}
+
+// the scatter of a stage and its probe partial sums
+int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStream_t stream) {
+  const int pix_blocks = (pa.S * pa.S + 255) / 256, nchunk = probe_nchunk(pa.B);
+  if (!scatter_in_range(g.B, g.S)) {
+    int rc = launch_scatter(g, stream);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_probe_partial, dim3(pix_blocks, nchunk), dim3(256), 0, stream, pa);
+    return check_launch("k_probe_partial");
+  }
+  const ScatterPlan plan = scatter_plan(g.Px, g.Py);
+  const int ns = scatter_blocks(g.Px, g.Py);
+  const dim3 grid(ns + pix_blocks * nchunk), blk(256);
+  if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter_probe<1>, grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  else hipLaunchKernelGGL(k_scatter_probe<4>, grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  return check_launch("k_scatter_probe");
 }
 
 int launch_probe_update(cf* probe, const cf* chi, const cf* obj, int Px, int Py, const float* pos, int N,
@@ -1978,7 +2033,7 @@ WsLayout layout(const pty_problem& p, const pty_gd_params& q, bool positions = f
   L.err = o; o = align256(o + (size_t)p.N * 8);
   L.grad = o; o = align256(o + npix * 8);
   L.spsum = o; o = align256(o + npix * 4);
-  L.tilemax = o; o = align256(o + (size_t)num_tiles(p.Px, p.Py) * 4);
+  L.tilemax = o; o = align256(o + (size_t)scatter_num_tiles(p.Px, p.Py) * 4);
   L.ppart = o; o = align256(o + (q.fix_probe ? 0 : probe_ws_bytes(p.S, q.max_batch)));
   L.cpart = o; o = align256(o + (size_t)CONSTRAINT_BLOCKS * 16);
   L.run = o; o = align256(o + ((int)B < q.max_batch ? npix * 24 : 0));
@@ -2013,7 +2068,13 @@ int validate_problem(const pty_problem* p) {
 // process ends.  Host code must use the per-device address from
 // hipGetSymbolAddress, never the array's name.
 // ---------------------------------------------------------------------------
-static __device__ __align__(256) unsigned char scratch[PTY_NOALLOC_SCRATCH_BYTES];
+// SCRATCH_EXTRA: room beyond the documented size for the scatter's tile
+// maxima (scatter_num_tiles is up to eight times the 8 x 64 tiles that
+// fit_stage_to_scratch counts, so that it accepts what it always accepted):
+// 4 bytes per 64 pixels up to SCATTER_SMALL_PIXELS, per 256 beyond, of an
+// object that fits the scratch (under 2 M pixels), 31 KiB at most.
+constexpr size_t SCRATCH_EXTRA = 64 * 1024;
+static __device__ __align__(256) unsigned char scratch[PTY_NOALLOC_SCRATCH_BYTES + SCRATCH_EXTRA];
 
 namespace {
 
@@ -2046,9 +2107,11 @@ int fit_stage_to_scratch(const pty_problem& p, pty_gd_params& q) {
   pty_gd_params t = q;
   int s = (q.stage > 0 && q.stage < q.max_batch) ? stage_size(q) : q.max_batch;
   size_t need = 0;
+  const size_t extra = align256((size_t)scatter_num_tiles(p.Px, p.Py) * 4) -
+                       align256((size_t)gather_num_tiles(p.Px, p.Py) * 4);
   while (true) {
     t.stage = s >= q.max_batch ? 0 : s;
-    need = layout(p, t).total;
+    need = layout(p, t).total - extra;
     if (need <= (size_t)PTY_NOALLOC_SCRATCH_BYTES) {
       q.stage = t.stage;
       return PTY_OK;
@@ -2120,7 +2183,7 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
     pipe_lock = std::unique_lock<std::mutex>(pipe->mu);
   }
   const size_t stage_elems = (size_t)stage * p.S * p.S;
-  const int ntiles = num_tiles(p.Px, p.Py);
+  const int ntiles = scatter_num_tiles(p.Px, p.Py);
   const double norm = (double)(float)(p.mean_intensity * (float)p.N);
   bool phat_valid = false;
   // complex object with probe update: the object step carries the fft2 of
@@ -2164,15 +2227,12 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
           g.run_last = s0 + ns == nb;
         }
         if (q.fix_probe) {
-          if ((rc = launch_gather(g, p.Px, p.Py, gs))) return rc;
+          if ((rc = launch_scatter(g, gs))) return rc;
         } else {
           ProbePartialArgs pa{chi_k, obj, p.positions, ob + s0, p.N, ns, p.S, p.Px, p.Py,
                               ppart + (size_t)(s0 / PROBE_CHUNK) * p.S * p.S * 3};
           pa.object_pot = V;
-          const int pix_blocks = (p.S * p.S + 255) / 256;
-          hipLaunchKernelGGL(k_gather_probe, dim3(ntiles + pix_blocks * probe_nchunk(ns)), dim3(GATHER_THREADS), 0,
-                             gs, g, pa, ntiles, pix_blocks);
-          if ((rc = check_launch("k_gather_probe"))) return rc;
+          if ((rc = launch_scatter_probe(g, pa, gs))) return rc;
         }
         if (pipe && (rc = hip_check(hipEventRecord(pipe->scatter_done[k & 1], gs), "hipEventRecord"))) return rc;
       }
@@ -2273,7 +2333,7 @@ int proj_run(const pty_problem* problem, const pty_gd_params* params, const pty_
   const int stage = correct ? p.N : stage_size(q);
   cf* obj = (cf*)p.object;
   cf* probe = (cf*)p.probe;
-  const int ntiles = num_tiles(p.Px, p.Py);
+  const int ntiles = scatter_num_tiles(p.Px, p.Py);
   const double norm = (double)(float)(p.mean_intensity * (float)p.N);
   const size_t S2 = (size_t)p.S * p.S;
   // the reference's Python-float coefficients, rounded to float32 where they
@@ -2306,14 +2366,11 @@ int proj_run(const pty_problem* problem, const pty_gd_params* params, const pty_
         g.run_last = s0 + ns == p.N;
       }
       if (q.fix_probe) {
-        if ((rc = launch_gather(g, p.Px, p.Py, stream))) return rc;
+        if ((rc = launch_scatter(g, stream))) return rc;
       } else {  // scatter and probe partial sums in one launch
         ProbePartialArgs pa{ex, obj, p.positions, order + s0, p.N, ns, p.S, p.Px, p.Py,
                             ppart + (size_t)(s0 / PROBE_CHUNK) * S2 * 3};
-        const int pix_blocks = (p.S * p.S + 255) / 256;
-        hipLaunchKernelGGL(k_gather_probe, dim3(ntiles + pix_blocks * probe_nchunk(ns)), dim3(GATHER_THREADS), 0,
-                           stream, g, pa, ntiles, pix_blocks);
-        if ((rc = check_launch("k_gather_probe"))) return rc;
+        if ((rc = launch_scatter_probe(g, pa, stream))) return rc;
       }
     }
     valid = 1;
@@ -2372,7 +2429,7 @@ MixedLayout mixed_layout(const pty_problem& p, const pty_gd_params& q, int K, bo
   L.err = o; o = align256(o + (size_t)p.N * 8);
   L.grad = o; o = align256(o + K * npix * 8);
   L.spsum = o; o = align256(o + K * npix * 4);
-  L.tilemax = o; o = align256(o + (size_t)K * num_tiles(p.Px, p.Py) * 4);
+  L.tilemax = o; o = align256(o + (size_t)K * scatter_num_tiles(p.Px, p.Py) * 4);
   L.total = o; o = align256(o + npix * 4);
   L.bmax = o; o = align256(o + MIXED_BLOCKS * 4);
   L.pstride = q.fix_probe ? 0 : align256(probe_ws_bytes(p.S, q.max_batch));
@@ -2425,7 +2482,7 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
   cf* probe = (cf*)p.probe;
   const size_t S2 = (size_t)p.S * p.S;
   const long long npix = (long long)p.Px * p.Py;
-  const int ntiles = num_tiles(p.Px, p.Py);
+  const int ntiles = scatter_num_tiles(p.Px, p.Py);
   const int nblk = grid_for(npix, 256, MIXED_BLOCKS);
   const std::vector<int> batches = subdivide(p.N, q.max_batch);
   const double norm = (double)(float)(p.mean_intensity * (float)p.N);
@@ -2454,14 +2511,11 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
         g.Px = p.Px; g.Py = p.Py; g.tiles_y = gather_tiles_y(p.Py); g.grad = grad + (size_t)k * npix;
         g.spsum = spsum + (size_t)k * npix; g.tilemax = tilemax + (size_t)k * ntiles;
         if (q.fix_probe) {
-          if ((rc = launch_gather(g, p.Px, p.Py, stream))) return rc;
+          if ((rc = launch_scatter(g, stream))) return rc;
         } else {  // the mode's scatter and probe partial sums in one launch
           ProbePartialArgs pa{chi_k, obj, p.positions, ob, p.N, nb, p.S, p.Px, p.Py,
                               (double*)(ws + L.ppart + k * L.pstride)};
-          const int pix_blocks = (p.S * p.S + 255) / 256;
-          hipLaunchKernelGGL(k_gather_probe, dim3(ntiles + pix_blocks * probe_nchunk(nb)), dim3(GATHER_THREADS), 0,
-                             stream, g, pa, ntiles, pix_blocks);
-          if ((rc = check_launch("k_gather_probe"))) return rc;
+          if ((rc = launch_scatter_probe(g, pa, stream))) return rc;
         }
       }
       hipLaunchKernelGGL(k_mixed_overlap, dim3(nblk), dim3(256), 0, stream, spsum, K, npix, total, bmax);
@@ -2581,7 +2635,7 @@ int pty_scatter_patches(const void* ps, const void* chi, const float* positions,
   a.ps = (const cf*)ps; a.chi = (const cf*)chi; a.positions = positions; a.order = order;
   a.N = N; a.B = B; a.S = S; a.Px = Px; a.Py = Py; a.tiles_y = gather_tiles_y(Py);
   a.grad = (cf*)grad; a.spsum = spsum; a.tilemax = tilemax;
-  return launch_gather(a, Px, Py, st(stream));
+  return launch_scatter(a, st(stream));
 }
 
 int pty_object_update(void* object, const void* grad, const float* spsum, const float* tilemax, int ntiles, int Px,
@@ -2594,7 +2648,7 @@ int pty_object_update(void* object, const void* grad, const float* spsum, const 
 
 size_t pty_probe_partials_bytes(int S, int B) { return probe_ws_bytes(S, B); }
 
-int pty_scatter_num_tiles(int Px, int Py) { return gather_num_tiles(Px, Py); }
+int pty_scatter_num_tiles(int Px, int Py) { return scatter_num_tiles(Px, Py); }
 
 int pty_probe_update(void* probe, const void* chi, const void* object, int Px, int Py, const float* positions, int N,
                      const int* order, int B, int S, float step_size, float normalization_min, void* partials,
@@ -2736,7 +2790,7 @@ int pty_loss_gradients(const void* object, const void* probe, int Px, int Py, co
       g.ps = ps; g.chi = chi; g.positions = positions; g.order = order + start; g.N = N; g.B = nb; g.S = S;
       g.Px = Px; g.Py = Py; g.tiles_y = gather_tiles_y(Py); g.grad = nullptr; g.spsum = nullptr;
       g.tilemax = nullptr; g.acc = oacc;
-      if ((rc = launch_gather(g, Px, Py, stream))) return rc;
+      if ((rc = launch_scatter(g, stream))) return rc;
     }
     if (grad_probe) {
       a.chi_in = chi;
@@ -2807,7 +2861,8 @@ int pty_gd_run_noalloc(const pty_problem* problem, const pty_gd_params* params, 
   if ((rc = fit_stage_to_scratch(*problem, q))) return rc;
   void* ws = nullptr;
   if ((rc = scratch_pointer(&ws))) return rc;
-  return gd_run(problem, &q, nullptr, orders, errors, ws, (size_t)PTY_NOALLOC_SCRATCH_BYTES, st(stream));
+  return gd_run(problem, &q, nullptr, orders, errors, ws, (size_t)PTY_NOALLOC_SCRATCH_BYTES + SCRATCH_EXTRA,
+                st(stream));
 }
 
 size_t pty_gd_positions_workspace_bytes(const pty_problem* problem, const pty_gd_params* params) {
