@@ -44,12 +44,19 @@ struct __attribute__((aligned(8))) cf {
 PTY_HD cf mkcf(float x, float y) { cf r; r.x = x; r.y = y; return r; }
 PTY_HD cf cadd(cf a, cf b) { return mkcf(a.x + b.x, a.y + b.y); }
 PTY_HD cf csub(cf a, cf b) { return mkcf(a.x - b.x, a.y - b.y); }
-PTY_HD cf cmul(cf a, cf b) { return mkcf(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// Fused multiply-adds are written out wherever a product meets a sum in the
+// transforms and the pointwise steps between them: left to the compiler, the
+// choice of the fused operand differs from kernel to kernel, and with it the
+// last bit of results that two launch sequences must form alike.
+PTY_HD float fma32(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+PTY_HD cf cmul(cf a, cf b) { return mkcf(fma32(-a.y, b.y, a.x * b.x), fma32(a.y, b.x, a.x * b.y)); }
 // conj(a) * b
-PTY_HD cf cconjmul(cf a, cf b) { return mkcf(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x); }
+PTY_HD cf cconjmul(cf a, cf b) { return mkcf(fma32(a.y, b.y, a.x * b.x), fma32(-a.y, b.x, a.x * b.y)); }
 PTY_HD cf cscale(cf a, float s) { return mkcf(a.x * s, a.y * s); }
 PTY_HD cf cconj(cf a) { return mkcf(a.x, -a.y); }
-PTY_HD float cabs2(cf a) { return a.x * a.x + a.y * a.y; }
+PTY_HD float cabs2(cf a) { return fma32(a.y, a.y, a.x * a.x); }
+// a + s * b
+PTY_HD cf caxpy(float s, cf b, cf a) { return mkcf(fma32(s, b.x, a.x), fma32(s, b.y, a.y)); }
 // conj(a) * b and |a|^2 with every product rounded to float32 before the
 // sum (no fused multiply-add), as NumPy's complex64 arithmetic forms them
 PTY_HD cf cconjmul_rn(cf a, cf b) {
@@ -120,29 +127,53 @@ template <bool INV> PTY_HD void dft4(cf& x0, cf& x1, cf& x2, cf& x3) {
   x3 = csub(t1, t3);
 }
 
+// Twiddles of the composite transforms, up to a positive real factor that the
+// next butterfly takes into its multiply-adds: two operations per twiddle
+// instead of four.
+// a * W8 / c, c = cos(pi/4)
+template <bool INV> PTY_HD cf tw8(cf a) { return INV ? mkcf(a.x - a.y, a.y + a.x) : mkcf(a.x + a.y, a.y - a.x); }
+// a * W8^3 / c
+template <bool INV> PTY_HD cf tw83(cf a) { return INV ? mkcf(-a.x - a.y, a.x - a.y) : mkcf(a.y - a.x, -a.x - a.y); }
+// a * W16 / cos(pi/8)
+template <bool INV> PTY_HD cf tw16(cf a) {
+  const float t = INV ? -0.41421356237309503f : 0.41421356237309503f;  // tan(pi/8)
+  return mkcf(fma32(t, a.y, a.x), fma32(-t, a.x, a.y));
+}
+// a * W16^3 / cos(pi/8)
+template <bool INV> PTY_HD cf tw163(cf a) {
+  const float t = 0.41421356237309503f;
+  return INV ? mkcf(fma32(t, a.x, -a.y), fma32(t, a.y, a.x)) : mkcf(fma32(t, a.x, a.y), fma32(t, a.y, -a.x));
+}
+
+// e + c o and e - c o into x[k], x[k + 4]
 template <bool INV> PTY_HD void dft8(cf* x) {
   const float c = 0.70710678118654752f;
   cf e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
   cf o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
   dft4<INV>(e0, e1, e2, e3);
   dft4<INV>(o0, o1, o2, o3);
-  // twiddles W8^k (forward: exp(-i pi k / 4))
-  cf w1 = INV ? mkcf(c * (o1.x - o1.y), c * (o1.x + o1.y)) : mkcf(c * (o1.x + o1.y), c * (o1.y - o1.x));
-  cf w2 = rot90<INV>(o2);
-  cf w3 = INV ? mkcf(-c * (o3.x + o3.y), c * (o3.x - o3.y)) : mkcf(c * (o3.y - o3.x), -c * (o3.x + o3.y));
+  const cf w1 = tw8<INV>(o1), w2 = rot90<INV>(o2), w3 = tw83<INV>(o3);
   x[0] = cadd(e0, o0); x[4] = csub(e0, o0);
-  x[1] = cadd(e1, w1); x[5] = csub(e1, w1);
+  x[1] = caxpy(c, w1, e1); x[5] = caxpy(-c, w1, e1);
   x[2] = cadd(e2, w2); x[6] = csub(e2, w2);
-  x[3] = cadd(e3, w3); x[7] = csub(e3, w3);
+  x[3] = caxpy(c, w3, e3); x[7] = caxpy(-c, w3, e3);
+}
+
+// outer butterfly of the 16-point transform: outputs k1, k1 + 4, ... from
+// t0 = a + C, t1 = a - C and s (b + d), s rot90(b - d)
+template <bool INV> PTY_HD void outer4(cf* x, int k1, cf t0, cf t1, cf sum, cf diff, float s) {
+  const cf r = rot90<INV>(diff);
+  x[k1] = caxpy(s, sum, t0);
+  x[k1 + 8] = caxpy(-s, sum, t0);
+  x[k1 + 4] = caxpy(s, r, t1);
+  x[k1 + 12] = caxpy(-s, r, t1);
 }
 
 // 16-point DFT as 4 x 4: inner DFT4 over n1 (stride 4), twiddle W16^(n2*k1),
-// outer DFT4 over n2.
+// outer DFT4 over n2.  144 operations (64 inner, 16 + 22 + 20 + 22 outer).
 template <bool INV> PTY_HD void dft16(cf* x) {
   const float c1 = 0.92387953251128676f;  // cos(pi/8)
-  const float s1 = 0.38268343236508977f;  // sin(pi/8)
   const float c2 = 0.70710678118654752f;
-  const float sg = INV ? 1.f : -1.f;      // sign of the twiddle angle
   cf y[16];
 #pragma unroll
   for (int n2 = 0; n2 < 4; ++n2) {
@@ -150,27 +181,22 @@ template <bool INV> PTY_HD void dft16(cf* x) {
     dft4<INV>(a, b, cc, d);
     y[n2 * 4 + 0] = a; y[n2 * 4 + 1] = b; y[n2 * 4 + 2] = cc; y[n2 * 4 + 3] = d;
   }
-  // W16^m for m = n2*k1 in {1,2,3,2,4,6,3,6,9}
-  const float wc[10] = {1.f, c1, c2, s1, 0.f, -s1, -c2, -c1, -1.f, -c1};
-  const float ws[10] = {0.f, s1, c2, c1, 1.f, c1, c2, s1, 0.f, -s1};
-#pragma unroll
-  for (int n2 = 1; n2 < 4; ++n2) {
-#pragma unroll
-    for (int k1 = 1; k1 < 4; ++k1) {
-      const int m = n2 * k1;
-      if (m == 4) {  // W16^4 is the quarter turn: a swap and a sign
-        y[n2 * 4 + k1] = rot90<INV>(y[n2 * 4 + k1]);
-      } else {
-        cf w = mkcf(wc[m], sg * ws[m]);
-        y[n2 * 4 + k1] = cmul(y[n2 * 4 + k1], w);
-      }
-    }
-  }
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    cf a = y[k1], b = y[4 + k1], cc = y[8 + k1], d = y[12 + k1];
+  {  // k1 = 0
+    cf a = y[0], b = y[4], cc = y[8], d = y[12];
     dft4<INV>(a, b, cc, d);
-    x[k1] = a; x[k1 + 4] = b; x[k1 + 8] = cc; x[k1 + 12] = d;
+    x[0] = a; x[4] = b; x[8] = cc; x[12] = d;
+  }
+  {  // k1 = 1: W, W^2, W^3
+    const cf b = tw16<INV>(y[5]), cc = tw8<INV>(y[9]), d = tw163<INV>(y[13]);
+    outer4<INV>(x, 1, caxpy(c2, cc, y[1]), caxpy(-c2, cc, y[1]), cadd(b, d), csub(b, d), c1);
+  }
+  {  // k1 = 2: W^2, W^4 (a quarter turn), W^6
+    const cf b = tw8<INV>(y[6]), cc = rot90<INV>(y[10]), d = tw83<INV>(y[14]);
+    outer4<INV>(x, 2, cadd(y[2], cc), csub(y[2], cc), cadd(b, d), csub(b, d), c2);
+  }
+  {  // k1 = 3: W^3, W^6, W^9 = -W
+    const cf b = tw163<INV>(y[7]), cc = tw83<INV>(y[11]), d = tw16<INV>(y[15]);
+    outer4<INV>(x, 3, caxpy(c2, cc, y[3]), caxpy(-c2, cc, y[3]), csub(b, d), cadd(b, d), c1);
   }
 }
 
@@ -677,10 +703,9 @@ template <int S> struct Fused {
       // place of F/|F|; a NaN far field stays NaN.  Selects, not a branch.
       const bool nz = m2 != 0.f;
       const float inv = nz ? frsq(m2) : 0.f;
-      const float mag = m2 * inv;
       const float ux = nz ? f.x * inv : 1.f, uy = f.y * inv;
-      const cf g = PROJ ? mkcf(amp * ux, amp * uy) : mkcf(amp * ux - f.x, amp * uy - f.y);
-      const float d = amp - mag;
+      const cf g = PROJ ? mkcf(amp * ux, amp * uy) : mkcf(fma32(amp, ux, -f.x), fma32(amp, uy, -f.y));
+      const float d = fma32(-m2, inv, amp);  // A - |F|
       acc += (double)(d * d);
       r.v[j] = MASK ? cscale(g, mj) : g;
     }

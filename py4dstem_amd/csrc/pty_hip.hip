@@ -10,10 +10,12 @@
 //                    work-group barriers (nine per position).
 //   k_scatter        one work group per object tile: float64 sums of the
 //                    staged patches in batch order (pty_scatter.inc).
-//   k_object_update  normalised object step.
-//   k_probe_partial / k_probe_update   probe step from staged terms.
-//   k_constraint_*   per-iteration object constraints; k_probe_com probe
-//                    recentring; k_error_reduce per-iteration error.
+//   k_scatter_probe  the scatter and the probe's chunk sums in one launch.
+//   k_update_reduce  normalised object step beside the probe's reduction;
+//   k_probe_apply*   probe step and fft2 of the new probe.
+//   k_iteration_sums, k_constraint_fft   end of an iteration: error, probe
+//                    recentring and constraint sums; then the object
+//                    constraints and fft2 of the recentred probe.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -376,6 +378,29 @@ __global__ __launch_bounds__(256) void k_acc_to_c64(const double* __restrict__ a
 //   forward: natural in -> natural (or kernel-layout) out
 //   inverse: natural (or kernel-layout) in -> natural out, scaled 1/S^2
 // ---------------------------------------------------------------------------
+// last row pass of a forward transform, kernel layout out through the frame:
+// a thread's own 16 elements are 128 contiguous bytes, which would make every
+// store instruction touch 64 cache lines; pieces of two elements per lane are
+// contiguous
+template <int S>
+__device__ __forceinline__ void fft2_rowB_store(int tid, typename Fused<S>::Regs& r, LdsPtr lds, const cf* tw,
+                                                cf* __restrict__ dst) {
+  using F = Frame<S>;
+  const int rr = F::row_line(tid), t = F::row_q(tid);
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) r.v[j] = lds.ld(F::at(rr, F::N1 * t + j));
+  Pass<S>::template B<false>(t, r.v, tw);
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) lds.st(F::at(rr, F::N1 * t + j), r.v[j]);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < F::N1 / 2; ++k) {
+    const int e = 2 * (k * F::T + tid);
+    dst[e] = lds.ld(F::at(e / S, e % S));
+    dst[e + 1] = lds.ld(F::at(e / S, e % S) + 1);
+  }
+}
+
 template <int S, bool INV>
 __device__ __forceinline__ void fft2_body(const cf* __restrict__ in, cf* __restrict__ out, int natural_io,
                                           int blk) {
@@ -402,27 +427,16 @@ __device__ __forceinline__ void fft2_body(const cf* __restrict__ in, cf* __restr
     __syncthreads();
     K::template p_rowA<false>(tid, r, lds, tw);
     wave_sync();
-    const int rr = F::row_line(tid), t = F::row_q(tid);
-#pragma unroll
-    for (int j = 0; j < F::N1; ++j) r.v[j] = lds.ld(F::at(rr, F::N1 * t + j));
-    Pass<S>::template B<false>(t, r.v, tw);
     if (natural_io) {
+      const int rr = F::row_line(tid), t = F::row_q(tid);
+#pragma unroll
+      for (int j = 0; j < F::N1; ++j) r.v[j] = lds.ld(F::at(rr, F::N1 * t + j));
+      Pass<S>::template B<false>(t, r.v, tw);
       const int kr = F::kidx(rr);
 #pragma unroll
       for (int j = 0; j < F::N1; ++j) dst[kr * S + F::kidx(F::N1 * t + j)] = r.v[j];
     } else {
-      // kernel layout out through the frame: a thread's own 16 elements are
-      // 128 contiguous bytes, which would make every store instruction touch
-      // 64 cache lines; pieces of two elements per lane are contiguous
-#pragma unroll
-      for (int j = 0; j < F::N1; ++j) lds.st(F::at(rr, F::N1 * t + j), r.v[j]);
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < F::N1 / 2; ++k) {
-        const int e = 2 * (k * F::T + tid);
-        dst[e] = lds.ld(F::at(e / S, e % S));
-        dst[e + 1] = lds.ld(F::at(e / S, e % S) + 1);
-      }
+      fft2_rowB_store<S>(tid, r, lds, tw, dst);
     }
   } else {
     const int rr = F::row_line(tid), t = F::row_q(tid);
@@ -512,18 +526,6 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather(GatherArgs a, int nti
 
 #include "pty_scatter.inc"
 
-__device__ float block_max(float v, float* sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] = fmaxf(sh[threadIdx.x], sh[threadIdx.x + s]);
-    __syncthreads();
-  }
-  float m = sh[0];
-  __syncthreads();
-  return m;
-}
-
 // Correctly rounded float32 square root of x >= 0 (IEEE / NumPy semantics).
 // The hardware estimate r is within one ulp.  The midpoints between r and its
 // float neighbours have at most 25 significant bits, so their squares are
@@ -555,89 +557,89 @@ __device__ __forceinline__ cf update_value(cf o, cf g, float nrm, float step, in
   return replace ? mkcf(g.x * nrm, g.y * nrm) : step_add(o, g, nrm, step);
 }
 
-__device__ __forceinline__ void object_update_body(cf* __restrict__ obj, const cf* __restrict__ grad,
-                                                   const float* __restrict__ spsum,
-                                                   const float* __restrict__ tilemax, int ntiles,
-                                                   long long npix, float step, float c1, float c2, int blk,
-                                                   int nblk, int replace = 0) {
-  __shared__ float sh[256];
-  float m = 0.f;
-  for (int i = threadIdx.x; i < ntiles; i += blockDim.x) m = fmaxf(m, tilemax[i]);
-  m = block_max(m, sh);
-  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < npix; p += (long long)nblk * blockDim.x) {
-    obj[p] = update_value(obj[p], grad[p], overlap_norm(spsum[p], m, c1, c2), step, replace);
-  }
+// maximum over the work group (waves by butterfly, then the waves' maxima;
+// every thread returns it); red: one word per wave
+__device__ __forceinline__ float group_max(float v, float* red) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float m = red[0];
+  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, red[w]);
+  return m;
 }
+
+struct ObjectUpdate {
+  cf* obj;              // complex object, or null with pot
+  float* pot;           // potential V
+  const cf* grad;
+  const float* spsum;
+  const float* tilemax;
+  int ntiles;
+  long long npix;
+  float step, c1, c2;
+  int replace;
+};
 
 // potential object (ptychographic_methods.py:1868-1880): V += step * (R * n),
 // R = Re(-i conj(exp(i V)) G) = cos V Im G - sin V Re G with G the float64
 // scatter of conj(P_shift) chi (conj(exp(i V)) is common to a pixel's terms;
 // the reference rounds each term's real part to float32 before its float64
 // sum, a difference at float32 rounding level)
-__global__ __launch_bounds__(256) void k_object_update_potential(float* __restrict__ V, const cf* __restrict__ grad,
-                                                                 const float* __restrict__ spsum,
-                                                                 const float* __restrict__ tilemax, int ntiles,
-                                                                 long long npix, float step, float c1, float c2) {
+__device__ __forceinline__ float potential_value(float v, cf g, float n, float step) {
 #pragma clang fp contract(off)
-  __shared__ float sh[256];
+  const cf o = expi(v);
+  const float R = (float)((double)o.x * (double)g.y - (double)o.y * (double)g.x);
+  return v + step * (R * n);
+}
+
+// work group blk of nblk (any multiple of 64 threads up to 1024).  The first
+// two pixels' values are requested ahead of the maximum over the tiles.
+__device__ __forceinline__ void object_update_body(const ObjectUpdate& u, int blk, int nblk) {
+  constexpr int N = 2;
+  __shared__ float red[16];
+  const long long stride = (long long)nblk * blockDim.x;
+  long long p = (long long)blk * blockDim.x + threadIdx.x;
+  float s[N], v[N];
+  cf g[N], o[N];
+  const auto load = [&]() {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const long long i = p + k * stride;
+      if (i >= u.npix) continue;
+      s[k] = u.spsum[i];
+      g[k] = u.grad[i];
+      if (u.pot) v[k] = u.pot[i];
+      else o[k] = u.obj[i];
+    }
+  };
+  load();
   float m = 0.f;
-  for (int i = threadIdx.x; i < ntiles; i += blockDim.x) m = fmaxf(m, tilemax[i]);
-  m = block_max(m, sh);
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    const float v = V[p];
-    const cf o = expi(v);
-    const cf g = grad[p];
-    const float R = (float)((double)o.x * (double)g.y - (double)o.y * (double)g.x);
-    const float n = overlap_norm(spsum[p], m, c1, c2);
-    V[p] = v + step * (R * n);
+  for (int i = threadIdx.x; i < u.ntiles; i += blockDim.x) m = fmaxf(m, u.tilemax[i]);
+  m = group_max(m, red);
+  while (p < u.npix) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const long long i = p + k * stride;
+      if (i >= u.npix) continue;
+      const float n = overlap_norm(s[k], m, u.c1, u.c2);
+      if (u.pot) u.pot[i] = potential_value(v[k], g[k], n, u.step);
+      else u.obj[i] = update_value(o[k], g[k], n, u.step, u.replace);
+    }
+    p += N * stride;
+    load();
   }
 }
 
-__global__ __launch_bounds__(256) void k_object_update(cf* __restrict__ obj, const cf* __restrict__ grad,
-                                                       const float* __restrict__ spsum,
-                                                       const float* __restrict__ tilemax, int ntiles,
-                                                       long long npix, float step, float c1, float c2,
-                                                       int replace) {
-  object_update_body(obj, grad, spsum, tilemax, ntiles, npix, step, c1, c2, blockIdx.x, gridDim.x, replace);
-}
-
-// the object step of a mini-batch and, in work group 0 of the same launch,
-// fft2 of the just-updated probe for the next mini-batch's fused pass (the
-// two are independent; the same arithmetic as k_object_update and k_fft2)
-template <int S>
-__global__ __launch_bounds__(Frame<S>::T) void k_object_update_fft(cf* __restrict__ obj, const cf* __restrict__ grad,
-                                                                  const float* __restrict__ spsum,
-                                                                  const float* __restrict__ tilemax, int ntiles,
-                                                                  long long npix, float step, float c1, float c2,
-                                                                  const cf* __restrict__ probe,
-                                                                  cf* __restrict__ phat) {
-  if (blockIdx.x == 0) {
-    fft2_body<S, false>(probe, phat, 0, 0);
-    return;
-  }
-  constexpr int T = Frame<S>::T;
-  __shared__ float sh[T];
-  const int tid = threadIdx.x;
-  float m = 0.f;
-  for (int i = tid; i < ntiles; i += T) m = fmaxf(m, tilemax[i]);
-  sh[tid] = m;
-  __syncthreads();
-  for (int s = T / 2; s > 0; s >>= 1) {
-    if (tid < s) sh[tid] = fmaxf(sh[tid], sh[tid + s]);
-    __syncthreads();
-  }
-  m = sh[0];
-  const long long nblk = gridDim.x - 1;
-  for (long long p = (long long)(blockIdx.x - 1) * T + tid; p < npix; p += nblk * T)
-    obj[p] = update_value(obj[p], grad[p], overlap_norm(spsum[p], m, c1, c2), step, 0);
+__global__ __launch_bounds__(1024) void k_object_update(ObjectUpdate u) {
+  object_update_body(u, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // mixed state (ptychographic_methods.py:2945-2975): the mode overlaps summed
 // in float32, modes in order, with a per-block maximum
 __global__ __launch_bounds__(256) void k_mixed_overlap(const float* __restrict__ spsum, int K, long long npix,
                                                        float* __restrict__ total, float* __restrict__ bmax) {
-  __shared__ float sh[256];
+  __shared__ float sh[16];
   float m = 0.f;
   for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
        p += (long long)gridDim.x * blockDim.x) {
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(256) void k_mixed_overlap(const float* __restrict__
     total[p] = s;
     m = fmaxf(m, s);
   }
-  m = block_max(m, sh);
+  m = group_max(m, sh);
   if (threadIdx.x == 0) bmax[blockIdx.x] = m;
 }
 
@@ -656,10 +658,10 @@ __global__ __launch_bounds__(256) void k_mixed_object_update(cf* __restrict__ ob
                                                              const float* __restrict__ bmax, int nblk,
                                                              long long npix, float step, float c1, float c2) {
 #pragma clang fp contract(off)
-  __shared__ float sh[256];
+  __shared__ float sh[16];
   float m = 0.f;
   for (int i = threadIdx.x; i < nblk; i += blockDim.x) m = fmaxf(m, bmax[i]);
-  m = block_max(m, sh);
+  m = group_max(m, sh);
   for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
        p += (long long)gridDim.x * blockDim.x) {
     float ux = 0.f, uy = 0.f;
@@ -695,18 +697,43 @@ struct ProbePartialArgs {
   const float* object_pot = nullptr;  // potential V: the patch is exp(i V)
 };
 
-// Sums over the chunk's slots, in batch order: conj(O) * chi (float32 products
-// rounded separately, float64 sums) and |O|^2 (squares and sums in float64,
-// two fused multiply-adds: no square root and no float32 rounding, which a
-// |O| in float32 would cost).
-__device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, int blk, int chunk) {
+// Sums over the chunk's slots: conj(O) * chi (float32 products rounded
+// separately, float64 sums) and |O|^2 (squares and sums in float64, two fused
+// multiply-adds: no square root and no float32 rounding, which a |O| in
+// float32 would cost).  The four waves of a work group take a quarter of the
+// chunk each (batch order inside a quarter) and the quarters are added in
+// order.  A lane holds R pixels: R = 1 gives four times the work groups, each
+// a chain of 16 slots, where small frames or few chunks would leave the chip
+// idle; R = 4 spreads a work group's set-up over more pixels.  The sums are
+// the same.  Measured with the scatter in the same launch: 507 slots of 64 px
+// 43 -> 17 us (potential object, R = 1 against a chain of 64 slots); 1024
+// slots of 128 px on 720^2 95 us with R = 1, 90 us with R = 4.
+constexpr int PROBE_GROUP = PROBE_CHUNK / 4;  // slots per wave
+constexpr int PROBE_PIX = 64;                 // pixels per work group at R = 1
+
+// R = 4 from this many R = 1 work groups on (four per CU)
+constexpr int PROBE_WIDE_GROUPS = 1024;
+__host__ __device__ inline int probe_pixels_per_lane(int S, int nchunk) {
+  return S * S / PROBE_PIX * nchunk > PROBE_WIDE_GROUPS ? 4 : 1;
+}
+
+template <int R> struct ProbeShared {
+  int2 anchor[PROBE_CHUNK];
+  double quarter[3][3][R * 64];
+};
+
+template <int R>
+__device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, int blk, int chunk,
+                                                   ProbeShared<R>& sh) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-  __shared__ int2 anchor[PROBE_CHUNK];
+  constexpr int U = 8 / R;  // slots loaded ahead of their sums
   const int S = a.S;
   const int b0 = chunk * PROBE_CHUNK;
-  if (b0 >= a.B) return;  // uniform over the work group
+  // uniform over the work group; the batched runner's grid covers its largest
+  // frame, so smaller frames get pixel blocks beyond theirs
+  if (b0 >= a.B || blk * (R * 64) >= S * S) return;
   const int nb = min(a.B - b0, PROBE_CHUNK);
   // the object index of the chunk's window origins (window rows and columns
   // in ascending order, origin S/2 before the patch anchor), once per work
@@ -714,65 +741,100 @@ __device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, in
   for (int t = threadIdx.x; t < nb; t += blockDim.x) {
     int idx = a.order[b0 + t];
     idx = ((unsigned)idx < (unsigned)a.N) ? idx : 0;
-    anchor[t] = make_int2(wrap1(wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px) - S / 2, a.Px),
-                          wrap1(wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py) - S / 2, a.Py));
+    sh.anchor[t] = make_int2(wrap1(wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px) - S / 2, a.Px),
+                             wrap1(wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py) - S / 2, a.Py));
   }
   __syncthreads();
-  const int pix = blk * blockDim.x + threadIdx.x;
-  if (pix >= S * S) return;
-  // window coordinates of probe pixel (i, j): corner-centred index ^ S/2
-  const unsigned wi = (unsigned)(pix / S) ^ (unsigned)(S / 2), wj = (unsigned)(pix % S) ^ (unsigned)(S / 2);
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int pix = blk * (R * 64) + lane;  // and 64 r beyond; S * S is a multiple of 256
   const unsigned Px = a.Px, Py = a.Py;
   const cf* chi = a.chi + (size_t)b0 * S * S + pix;
-  double re = 0.0, im = 0.0, so = 0.0;
-  const auto object = [&](int k) {
-    const int2 w = anchor[k];
-    unsigned r = (unsigned)w.x + wi, q = (unsigned)w.y + wj;
-    r = umin(r, r - Px);  // origin and window coordinate below Px: one wrap
-    q = umin(q, q - Py);
-    return a.object_pot ? expi(elem(a.object_pot, r * Py + q)) : elem(a.object, r * Py + q);
-  };
-  const auto add = [&](cf o, cf c) {
-    const double x = o.x, y = o.y;
-    so = __builtin_fma(x, x, so);
-    so = __builtin_fma(y, y, so);
-    const cf g = cconjmul_rn(o, c);
-    re += (double)g.x;
-    im += (double)g.y;
-  };
-  constexpr int U = 8;  // slots loaded ahead of their sums
-  int k = 0;
-  for (; k + U <= nb; k += U) {
-    cf o[U], c[U];
+  // window coordinates of probe pixel (i, j): corner-centred index ^ S/2
+  unsigned wi[R], wj[R];
+  double re[R], im[R], so[R];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      o[u] = object(k + u);
-      c[u] = elem(chi, (unsigned)(k + u) * (unsigned)(S * S));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) add(o[u], c[u]);
+  for (int r = 0; r < R; ++r) {
+    wi[r] = (unsigned)((pix + 64 * r) >> __builtin_ctz(S)) ^ (unsigned)(S / 2);  // S a power of two
+    wj[r] = (unsigned)((pix + 64 * r) & (S - 1)) ^ (unsigned)(S / 2);
+    re[r] = im[r] = so[r] = 0.0;
   }
-  for (; k < nb; ++k) add(object(k), elem(chi, (unsigned)k * (unsigned)(S * S)));
-  double* p = a.part + ((size_t)chunk * S * S + pix) * 3;
-  p[0] = re;
-  p[1] = im;
-  p[2] = so;
+  const auto object = [&](int k, int r) {
+    const int2 w = sh.anchor[k];
+    unsigned x = (unsigned)w.x + wi[r], y = (unsigned)w.y + wj[r];
+    x = umin(x, x - Px);  // origin and window coordinate below Px: one wrap
+    y = umin(y, y - Py);
+    return a.object_pot ? expi(elem(a.object_pot, x * Py + y)) : elem(a.object, x * Py + y);
+  };
+  const auto add = [&](cf o, cf c, int r) {
+    const double x = o.x, y = o.y;
+    so[r] = __builtin_fma(x, x, so[r]);
+    so[r] = __builtin_fma(y, y, so[r]);
+    const cf t = cconjmul_rn(o, c);
+    re[r] += (double)t.x;
+    im[r] += (double)t.y;
+  };
+  int k = g * PROBE_GROUP;
+  const int k1 = min(nb, k + PROBE_GROUP);
+  for (; k + U <= k1; k += U) {
+    cf o[U][R], c[U][R];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        o[u][r] = object(k + u, r);
+        c[u][r] = elem(chi, (unsigned)(k + u) * (unsigned)(S * S) + 64 * r);
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) add(o[u][r], c[u][r], r);
+  }
+  for (; k < k1; ++k)
+#pragma unroll
+    for (int r = 0; r < R; ++r) add(object(k, r), elem(chi, (unsigned)k * (unsigned)(S * S) + 64 * r), r);
+  if (g > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      sh.quarter[g - 1][0][64 * r + lane] = re[r];
+      sh.quarter[g - 1][1][64 * r + lane] = im[r];
+      sh.quarter[g - 1][2][64 * r + lane] = so[r];
+    }
+  }
+  __syncthreads();
+  if (g > 0) return;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      re[r] += sh.quarter[h][0][64 * r + lane];
+      im[r] += sh.quarter[h][1][64 * r + lane];
+      so[r] += sh.quarter[h][2][64 * r + lane];
+    }
+    double* p = a.part + ((size_t)chunk * S * S + pix + 64 * r) * 3;
+    p[0] = re[r];
+    p[1] = im[r];
+    p[2] = so[r];
+  }
 }
 
 __global__ __launch_bounds__(256) void k_probe_partial(ProbePartialArgs a) {
-  probe_partial_body(a, blockIdx.x, blockIdx.y);
+  __shared__ ProbeShared<4> sh;
+  probe_partial_body<4>(a, blockIdx.x, blockIdx.y, sh);
 }
 
 // the scatter of a stage (work groups [0, nscatter)) and its probe partial
 // sums (the rest, pixel block fastest) in one launch: both only read the
 // fused pass's staged terms
-template <int R>
+template <int R, int RP>
 __global__ __launch_bounds__(256) void k_scatter_probe(GatherArgs g, ScatterPlan plan, int nscatter,
                                                        ProbePartialArgs pa, int pix_blocks) {
-  __shared__ ScatterShared<R> sh;
+  __shared__ union {
+    ScatterShared<R> scatter;
+    ProbeShared<RP> probe;
+  } sh;
   const int b = (int)blockIdx.x;
-  if (b < nscatter) scatter_body<R>(g, plan, b, sh);
-  else probe_partial_body(pa, (b - nscatter) % pix_blocks, (b - nscatter) / pix_blocks);
+  if (b < nscatter) scatter_body<R>(g, plan, b, sh.scatter);
+  else probe_partial_body<RP>(pa, (b - nscatter) % pix_blocks, (b - nscatter) / pix_blocks, sh.probe);
 }
 
 // per-pixel sum of the chunk partials: PROBE_REDUCE_GROUPS contiguous chunk
@@ -828,46 +890,185 @@ __device__ __forceinline__ void probe_reduce_body(const double* __restrict__ par
   if (threadIdx.x == 0) bmax[blk] = sh[0];
 }
 
-__global__ __launch_bounds__(PROBE_REDUCE_THREADS) void k_probe_reduce(const double* __restrict__ part, int nchunk,
-                                                      int npix, cf* __restrict__ gsum,
-                                                      float* __restrict__ osum,
-                                                      float* __restrict__ bmax) {
-  probe_reduce_body(part, nchunk, npix, gsum, osum, bmax, blockIdx.x);
+struct ProbeStep {
+  const double* part;  // chunk partials
+  int nchunk, npix;
+  cf* gsum;
+  float* osum;
+  float* bmax;         // [npix / 256] maxima of osum
+  cf* probe;
+  float step, c1, c2;
+  int replace;
+};
+
+// the probe's chunk sums (work groups [0, npix / 256)) and the object step
+// (the rest) in one launch: both only read the scatter's and the probe
+// partials' results
+__global__ __launch_bounds__(PROBE_REDUCE_THREADS) void k_update_reduce(ProbeStep q, ObjectUpdate u) {
+  const int nred = q.npix / 256;
+  if ((int)blockIdx.x < nred) probe_reduce_body(q.part, q.nchunk, q.npix, q.gsum, q.osum, q.bmax, blockIdx.x);
+  else object_update_body(u, (int)blockIdx.x - nred, (int)gridDim.x - nred);
 }
 
-__device__ __forceinline__ void probe_apply_body(cf* __restrict__ probe, const cf* __restrict__ gsum,
-                                                 const float* __restrict__ osum, const float* __restrict__ bmax,
-                                                 int nblk, int npix, float step, float c1, float c2, int blk,
-                                                 int replace = 0) {
-  __shared__ float sh[256];
+// largest osum of the probe (every thread returns it)
+__device__ __forceinline__ float probe_max(const float* __restrict__ bmax, int nblk, float* red) {
   float m = 0.f;
   for (int i = threadIdx.x; i < nblk; i += blockDim.x) m = fmaxf(m, bmax[i]);
-  m = block_max(m, sh);
-  const int pix = blk * blockDim.x + threadIdx.x;
-  if (pix < npix) probe[pix] = update_value(probe[pix], gsum[pix], overlap_norm(osum[pix], m, c1, c2), step, replace);
+  return group_max(m, red);
 }
 
-__global__ __launch_bounds__(256) void k_probe_apply(cf* __restrict__ probe, const cf* __restrict__ gsum,
-                                                     const float* __restrict__ osum,
-                                                     const float* __restrict__ bmax, int nblk, int npix,
-                                                     float step, float c1, float c2, int replace) {
-  probe_apply_body(probe, gsum, osum, bmax, nblk, npix, step, c1, c2, blockIdx.x, replace);
+// the probe step of N pixels: all values requested ahead of the maximum,
+// results stored and left in v
+template <int N, class Pix>
+__device__ __forceinline__ void probe_values(const ProbeStep& q, Pix pix, float* red, cf* v) {
+  cf p[N], g[N];
+  float o[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    p[k] = q.probe[pix(k)];
+    g[k] = q.gsum[pix(k)];
+    o[k] = q.osum[pix(k)];
+  }
+  const float m = probe_max(q.bmax, q.npix / 256, red);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    v[k] = update_value(p[k], g[k], overlap_norm(o[k], m, q.c1, q.c2), q.step, q.replace);
+    q.probe[pix(k)] = v[k];
+  }
+}
+
+__device__ __forceinline__ void probe_apply_body(const ProbeStep& q, int blk) {
+  __shared__ float red[16];
+  const int pix = blk * blockDim.x + threadIdx.x;  // npix is a multiple of the work group
+  cf v;
+  probe_values<1>(q, [&](int) { return pix; }, red, &v);
+}
+
+__global__ __launch_bounds__(256) void k_probe_apply(ProbeStep q) { probe_apply_body(q, blockIdx.x); }
+
+// The probe step and fft2 of the new probe (kernel layout) for the next
+// mini-batch, frames of 32 and 64 px: one work group, the updated pixels go
+// from registers into the column passes.  At 128 px one work group takes
+// too long over the 16384 pixels (24 us measured): there the step and the
+// column transforms run on 16 work groups of 8 columns (k_probe_apply_cols)
+// and the row transforms on 16 of 8 rows (k_probe_rows).  The arithmetic is
+// that of k_probe_apply and k_fft2.
+template <int S> __global__ __launch_bounds__(Frame<S>::T) void k_probe_apply_fft(ProbeStep q, cf* __restrict__ phat) {
+  using F = Frame<S>;
+  using K = Fused<S>;
+  __shared__ cf lds_mem[F::LDS_WORDS];
+  __shared__ cf tw[K::TW_WORDS];
+  __shared__ float red[16];
+  const int tid = threadIdx.x;
+  K::twiddles(tid, LdsPtr{tw}, F::T);
+  LdsPtr lds{lds_mem};
+  typename K::Regs r;
+  const int cc = F::col_line(tid), n2 = F::col_q(tid);
+  // the barrier of its maximum publishes tw
+  probe_values<F::N1>(q, [&](int k) { return (n2 + F::N2 * k) * S + cc; }, red, r.v);
+  Pass<S>::template A<false>(n2, r.v, tw);
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) lds.st(F::at(n2 + F::N2 * k, cc), r.v[k]);
+  __syncthreads();
+  K::template p_colB<false>(tid, r, lds, tw);
+  __syncthreads();
+  K::template p_rowA<false>(tid, r, lds, tw);
+  wave_sync();
+  fft2_rowB_store<S>(tid, r, lds, tw, phat);
+}
+
+constexpr int PROBE_LINES = 8;  // columns or rows of a work group of the split transform
+
+// the step on all 256 threads (its square roots and divisions), the column
+// transforms on the first wave
+template <int S> __global__ __launch_bounds__(256) void k_probe_apply_cols(ProbeStep q, cf* __restrict__ phat) {
+  using F = Frame<S>;
+  using K = Fused<S>;
+  constexpr int P = PROBE_LINES + 1;
+  static_assert(PROBE_LINES * F::N2 == 64, "the transforms fill one wave");
+  __shared__ cf buf[S * P];
+  __shared__ cf tw[K::TW_WORDS];
+  __shared__ float red[16];
+  const int tid = threadIdx.x, c = tid % PROBE_LINES, n2 = tid / PROBE_LINES;
+  const int col = blockIdx.x * PROBE_LINES + c;
+  constexpr int N = S * PROBE_LINES / 256, ROWS = 256 / PROBE_LINES;
+  K::twiddles(tid, LdsPtr{tw}, 256);
+  cf v[F::N1];
+  probe_values<N>(q, [&](int k) { return (n2 + ROWS * k) * S + col; }, red, v);
+#pragma unroll
+  for (int k = 0; k < N; ++k) buf[(n2 + ROWS * k) * P + c] = v[k];
+  __syncthreads();
+  if (tid >= 64) return;
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) v[k] = buf[(n2 + F::N2 * k) * P + c];
+  Pass<S>::template A<false>(n2, v, tw);
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) buf[(n2 + F::N2 * k) * P + c] = v[k];
+  wave_sync();
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) v[j] = buf[(F::N1 * n2 + j) * P + c];
+  Pass<S>::template B<false>(n2, v, tw);
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) phat[(F::N1 * n2 + j) * S + col] = v[j];
+}
+
+// rows of the column-transformed probe, in place
+template <int S> __global__ __launch_bounds__(PROBE_LINES* Frame<S>::N2) void k_probe_rows(cf* __restrict__ phat) {
+  using F = Frame<S>;
+  using K = Fused<S>;
+  constexpr int T = PROBE_LINES * F::N2, PITCH = F::PITCH;
+  __shared__ cf buf[PROBE_LINES * PITCH];
+  __shared__ cf tw[K::TW_WORDS];
+  const int tid = threadIdx.x, l = tid / F::N2, n2 = tid % F::N2;
+  K::twiddles(tid, LdsPtr{tw}, T);
+  cf* rows = phat + blockIdx.x * PROBE_LINES * S;
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) {  // coalesced: element k T + tid of the eight rows
+    const int e = k * T + tid;
+    buf[(e / S) * PITCH + F::phys(e % S)] = rows[e];
+  }
+  __syncthreads();
+  cf* line = buf + l * PITCH;
+  cf v[F::N1];
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) v[k] = line[F::phys(n2 + F::N2 * k)];
+  Pass<S>::template A<false>(n2, v, tw);
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) line[F::phys(n2 + F::N2 * k)] = v[k];
+  wave_sync();
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) v[j] = line[F::phys(F::N1 * n2 + j)];
+  Pass<S>::template B<false>(n2, v, tw);
+#pragma unroll
+  for (int j = 0; j < F::N1; ++j) line[F::phys(F::N1 * n2 + j)] = v[j];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < F::N1; ++k) {
+    const int e = k * T + tid;
+    rows[e] = buf[(e / S) * PITCH + F::phys(e % S)];
+  }
 }
 
 // ---------------------------------------------------------------------------
 // constraints
 // ---------------------------------------------------------------------------
-constexpr int CONSTRAINT_BLOCKS = 256;
+// The masked sum is split the same way in every launch that forms it, whatever
+// its work-group size: CONSTRAINT_PARTS partial sums, part g over the pixels
+// g * 128 + t + k * 128 * CONSTRAINT_PARTS (t < 128), so a reconstruction's
+// result does not depend on which launch carried the sum.
+constexpr int CONSTRAINT_PARTS = 512;
 
-// masked sum of the phase (complex object) or of the potential (pot != null)
+// masked sum of the phase (complex object) or of the potential (pot != null);
+// work group blk of CONSTRAINT_PARTS / (blockDim / 128)
 __device__ __forceinline__ void constraint_partial_body(const cf* __restrict__ obj,
                                                         const unsigned char* __restrict__ mask, long long npix,
-                                                        double* part, int blk, int nblk,
-                                                        const float* __restrict__ pot = nullptr) {
-  __shared__ double ssum[256];
-  __shared__ double scnt[256];
+                                                        double* part, int blk, const float* __restrict__ pot) {
+  __shared__ double half[16][2];
+  const int wave = threadIdx.x >> 6, t = threadIdx.x & 127;
+  const int g = blk * (int)(blockDim.x >> 7) + (int)(threadIdx.x >> 7);
   double s = 0.0, c = 0.0;
-  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < npix; p += (long long)nblk * blockDim.x) {
+#pragma unroll 4
+  for (long long p = (long long)g * 128 + t; p < npix; p += 128 * CONSTRAINT_PARTS) {
     if (mask[p]) {
       if (pot) {
         s += (double)pot[p];
@@ -878,50 +1079,76 @@ __device__ __forceinline__ void constraint_partial_body(const cf* __restrict__ o
       c += 1.0;
     }
   }
-  ssum[threadIdx.x] = s;
-  scnt[threadIdx.x] = c;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off);
+    c += __shfl_xor(c, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    half[wave][0] = s;
+    half[wave][1] = c;
+  }
   __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) {
-      ssum[threadIdx.x] += ssum[threadIdx.x + k];
-      scnt[threadIdx.x] += scnt[threadIdx.x + k];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    part[2 * blk] = ssum[0];
-    part[2 * blk + 1] = scnt[0];
+  if (t == 0) {
+    part[2 * g] = half[wave][0] + half[wave + 1][0];
+    part[2 * g + 1] = half[wave][1] + half[wave + 1][1];
   }
 }
 
-__global__ __launch_bounds__(256) void k_constraint_partial(const cf* __restrict__ obj,
-                                                            const unsigned char* __restrict__ mask,
-                                                            long long npix, double* part,
-                                                            const float* __restrict__ pot) {
-  constraint_partial_body(obj, mask, npix, part, blockIdx.x, gridDim.x, pot);
-}
-
-__device__ __forceinline__ void constraint_apply_body(cf* __restrict__ obj, long long npix,
-                                                      const double* __restrict__ part, int nparts, int use_mask,
-                                                      float shrinkage_rad, int pure_phase, int blk, int nblk) {
+// total shrinkage of the constraint step (every thread returns it): one wave
+// adds the partial sums, eight per lane and then by butterfly (a single
+// thread adding them in turn took 20 us per launch)
+__device__ __forceinline__ float constraint_shrink(const double* __restrict__ part, int use_mask,
+                                                   float shrinkage_rad) {
   __shared__ float shrink_sh;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     float shrink = shrinkage_rad;
     if (use_mask) {
       double s = 0.0, c = 0.0;
-      for (int k = 0; k < nparts; ++k) {
-        s += part[2 * k];
-        c += part[2 * k + 1];
+#pragma unroll
+      for (int k = 0; k < CONSTRAINT_PARTS / 64; ++k) {
+        s += part[2 * (64 * k + threadIdx.x)];
+        c += part[2 * (64 * k + threadIdx.x) + 1];
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_xor(s, off);
+        c += __shfl_xor(c, off);
       }
       shrink = shrink + (float)(s / c);
     }
-    shrink_sh = shrink;
+    if (threadIdx.x == 0) shrink_sh = shrink;
   }
   __syncthreads();
-  const float shrink = shrink_sh;
-  const bool do_shrink = use_mask || shrinkage_rad > 0.f;
-  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < npix; p += (long long)nblk * blockDim.x) {
-    cf o = obj[p];
+  return shrink_sh;
+}
+
+struct ConstraintArgs {
+  cf* obj;                    // complex object, or null with pot
+  float* pot;                 // potential V
+  const unsigned char* mask;  // null: no baseline
+  long long npix;
+  double* part;               // [CONSTRAINT_PARTS][2]
+  float shrinkage_rad;
+  int pure_phase, positivity;
+};
+
+// complex object: shrinkage, then threshold (or pure phase).  Potential
+// (ptychographic_constraints.py:60-118, 447-462): V minus (shrinkage_rad +
+// masked mean of V) when shrinking, then clip at zero with positivity; NaN
+// stays NaN as under numpy clip.
+__device__ __forceinline__ void constraint_apply_body(const ConstraintArgs& a, int blk, int nblk) {
+  const float shrink = constraint_shrink(a.part, a.mask != nullptr, a.shrinkage_rad);
+  const bool do_shrink = a.mask != nullptr || a.shrinkage_rad > 0.f;
+  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < a.npix; p += (long long)nblk * blockDim.x) {
+    if (a.pot) {
+      float v = a.pot[p];
+      if (do_shrink) v = v - shrink;
+      if (a.positivity) v = v < 0.f ? 0.f : v;
+      a.pot[p] = v;
+      continue;
+    }
+    cf o = a.obj[p];
     if (do_shrink) {
       const float ph = atan2f(o.y, o.x) - shrink;
       const float am = hypot_f(o.x, o.y);
@@ -930,59 +1157,37 @@ __device__ __forceinline__ void constraint_apply_body(cf* __restrict__ obj, long
       o = mkcf(am * cs, am * sn);
     }
     const float ph = atan2f(o.y, o.x);
-    const float am = pure_phase ? 1.0f : fminf(hypot_f(o.x, o.y), 1.0f);
+    const float am = a.pure_phase ? 1.0f : fminf(hypot_f(o.x, o.y), 1.0f);
     float sn, cs;
     sincosf(ph, &sn, &cs);
-    obj[p] = mkcf(am * cs, am * sn);
+    a.obj[p] = mkcf(am * cs, am * sn);
   }
 }
 
-__global__ __launch_bounds__(256) void k_constraint_apply(cf* __restrict__ obj, long long npix,
-                                                          const double* __restrict__ part, int nparts,
-                                                          int use_mask, float shrinkage_rad,
-                                                          int pure_phase) {
-  constraint_apply_body(obj, npix, part, nparts, use_mask, shrinkage_rad, pure_phase, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(256) void k_constraint_partial(ConstraintArgs a) {
+  constraint_partial_body(a.obj, a.mask, a.npix, a.part, blockIdx.x, a.pot);
 }
 
-// potential object (ptychographic_constraints.py:60-118, 447-462): V minus
-// (shrinkage_rad + masked mean of V) when shrinking, then clip at zero when
-// object_positivity; NaN stays NaN as under numpy clip
-__global__ __launch_bounds__(256) void k_constraint_apply_potential(float* __restrict__ V, long long npix,
-                                                                    const double* __restrict__ part, int nparts,
-                                                                    int use_mask, float shrinkage_rad,
-                                                                    int positivity) {
-  __shared__ float shrink_sh;
-  if (threadIdx.x == 0) {
-    float shrink = shrinkage_rad;
-    if (use_mask) {
-      double s = 0.0, c = 0.0;
-      for (int k = 0; k < nparts; ++k) {
-        s += part[2 * k];
-        c += part[2 * k + 1];
-      }
-      shrink = shrink + (float)(s / c);
-    }
-    shrink_sh = shrink;
-  }
-  __syncthreads();
-  const float shrink = shrink_sh;
-  const bool do_shrink = use_mask || shrinkage_rad > 0.f;
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    float v = V[p];
-    if (do_shrink) v = v - shrink;
-    if (positivity) v = v < 0.f ? 0.f : v;
-    V[p] = v;
-  }
+__global__ __launch_bounds__(256) void k_constraint_apply(ConstraintArgs a) {
+  constraint_apply_body(a, blockIdx.x, gridDim.x);
 }
 
 // probe centre of mass (corner-centred coordinates) and Fourier recentring
+// |v|^2 (in float64: no square root, no rounding) and its moments
+__device__ __forceinline__ void com_terms(cf v, int fi, int fj, double& sI, double& sx, double& sy) {
+  const double x = v.x, y = v.y, I = __builtin_fma(y, y, x * x);
+  sI += I;
+  sx = __builtin_fma((double)fi, I, sx);
+  sy = __builtin_fma((double)fj, I, sy);
+}
+
 template <int S> __device__ __forceinline__ void probe_com_body(cf* __restrict__ probe) {
   using F = Frame<S>;
   using K = Fused<S>;
   constexpr int T = F::T;
   __shared__ cf lds_mem[F::LDS_WORDS];
   __shared__ cf tw[Fused<S>::TW_WORDS];
+  __shared__ cf ramp[2 * S];
   __shared__ double red[3][T / 64];
   __shared__ float shift[2];
   const int tid = threadIdx.x;
@@ -990,17 +1195,11 @@ template <int S> __device__ __forceinline__ void probe_com_body(cf* __restrict__
   LdsPtr lds{lds_mem};
   typename K::Regs r;
   const int cc = F::col_line(tid), n2 = F::col_q(tid);
+#pragma unroll
+  for (int m = 0; m < F::N1; ++m) r.v[m] = probe[(n2 + F::N2 * m) * S + cc];
   double sI = 0.0, sx = 0.0, sy = 0.0;
 #pragma unroll
-  for (int m = 0; m < F::N1; ++m) {
-    const int i = n2 + F::N2 * m;
-    r.v[m] = probe[i * S + cc];
-    const float a = hypot_f(r.v[m].x, r.v[m].y);
-    const double I = (double)(a * a);
-    sI += I;
-    sx += (double)F::fidx(i) * I;
-    sy += (double)F::fidx(cc) * I;
-  }
+  for (int m = 0; m < F::N1; ++m) com_terms(r.v[m], F::fidx(n2 + F::N2 * m), F::fidx(cc), sI, sx, sy);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     sI += __shfl_xor(sI, off);
@@ -1024,26 +1223,28 @@ template <int S> __device__ __forceinline__ void probe_com_body(cf* __restrict__
 #pragma unroll
   for (int m = 0; m < F::N1; ++m) lds.st(F::at(n2 + F::N2 * m, cc), r.v[m]);
   __syncthreads();
+  // the ramp of either axis, once per frequency (published by the next barrier)
+  for (int k = tid; k < 2 * S; k += T) ramp[k] = K::ramp1(k % S, shift[k / S]);
   K::template p_colB<false>(tid, r, lds, tw);
   __syncthreads();
   K::template p_rowA<false>(tid, r, lds, tw);
-  __syncthreads();
+  wave_sync();
   {
     const int rr = F::row_line(tid), t = F::row_q(tid);
 #pragma unroll
     for (int j = 0; j < F::N1; ++j) r.v[j] = lds.ld(F::at(rr, F::N1 * t + j));
     Pass<S>::template B<false>(t, r.v, tw);
-    const cf ex = K::ramp1(F::kidx(rr), shift[0]);
+    const cf ex = ramp[F::kidx(rr)];
 #pragma unroll
     for (int j = 0; j < F::N1; ++j) {
-      const cf e = cmul(ex, K::ramp1(F::kidx(F::N1 * t + j), shift[1]));
+      const cf e = cmul(ex, ramp[S + F::kidx(F::N1 * t + j)]);
       r.v[j] = cmul(r.v[j], e);
     }
     Pass<S>::template B<true>(t, r.v, tw);
 #pragma unroll
     for (int j = 0; j < F::N1; ++j) lds.st(F::at(rr, F::N1 * t + j), r.v[j]);
   }
-  __syncthreads();
+  wave_sync();
   K::template p_rowA<true>(tid, r, lds, tw);
   __syncthreads();
   K::template p_colB<true>(tid, r, lds, tw);
@@ -1072,12 +1273,7 @@ __global__ __launch_bounds__(Frame<S>::T) void k_probe_com_measure(const cf* __r
 #pragma unroll
   for (int m = 0; m < F::N1; ++m) {
     const int i = n2 + F::N2 * m;
-    const cf v = probe[i * S + cc];
-    const float a = hypot_f(v.x, v.y);
-    const double I = (double)(a * a);
-    sI += I;
-    sx += (double)F::fidx(i) * I;
-    sy += (double)F::fidx(cc) * I;
+    com_terms(probe[i * S + cc], F::fidx(i), F::fidx(cc), sI, sx, sy);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -1149,16 +1345,22 @@ __global__ __launch_bounds__(Frame<S>::T) void k_probe_shift_modes(cf* __restric
   for (int m = 0; m < F::N1; ++m) pk[(n2 + F::N2 * m) * S + cc] = r.v[m];
 }
 
-// per-iteration error: fixed-order float64 sum, normalised
+// per-iteration error: float64 sum, normalised, in the fixed order of 1024
+// strided sums and a tree over them whatever the work-group size
 __device__ __forceinline__ void error_reduce_body(const double* __restrict__ err, int n, double norm,
                                                   double* __restrict__ out) {
-  __shared__ double sh[1024];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) s += err[i];
-  sh[threadIdx.x] = s;
+  constexpr int V = 1024;
+  __shared__ double sh[V];
+  const int T = blockDim.x;
+  for (int v = threadIdx.x; v < V; v += T) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int i = v; i < n; i += V) s += err[i];
+    sh[v] = s;
+  }
   __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
+  for (int k = V / 2; k > 0; k >>= 1) {
+    for (int v = threadIdx.x; v < k; v += T) sh[v] += sh[v + k];
     __syncthreads();
   }
   if (threadIdx.x == 0) out[0] = sh[0] / norm;
@@ -1167,6 +1369,45 @@ __device__ __forceinline__ void error_reduce_body(const double* __restrict__ err
 __global__ __launch_bounds__(1024) void k_error_reduce(const double* __restrict__ err, int n,
                                                        double norm, double* __restrict__ out) {
   error_reduce_body(err, n, norm, out);
+}
+
+// ---------------------------------------------------------------------------
+// end of an iteration, two launches: the independent sums and the probe
+// recentring, then the object constraints and fft2 of the recentred probe for
+// the next iteration.  Each part is a few work groups of latency-bound work
+// (the recentring and the transform are one work group), so they share a
+// launch instead of following one another.
+// ---------------------------------------------------------------------------
+struct ErrorArgs {
+  const double* err;
+  int n;
+  double norm;
+  double* out;  // null: the error is not formed here
+};
+
+// work group 0: the error; 1: the probe recentring when `probe`; the rest
+// (when c.mask): the constraint's partial sums
+template <int S>
+__global__ __launch_bounds__(Frame<S>::T) void k_iteration_sums(ErrorArgs e, ConstraintArgs c, cf* probe) {
+  const int b = (int)blockIdx.x, first = probe ? 2 : 1;
+  if (b == 0) {
+    if (e.out) error_reduce_body(e.err, e.n, e.norm, e.out);
+  } else if (b < first) probe_com_body<S>(probe);
+  else constraint_partial_body(c.obj, c.mask, c.npix, c.part, b - first, c.pot);
+}
+
+// without the recentring (any frame size)
+__global__ __launch_bounds__(256) void k_iteration_sums_only(ErrorArgs e, ConstraintArgs c) {
+  if (blockIdx.x == 0) {
+    if (e.out) error_reduce_body(e.err, e.n, e.norm, e.out);
+  } else constraint_partial_body(c.obj, c.mask, c.npix, c.part, (int)blockIdx.x - 1, c.pot);
+}
+
+// work group 0: fft2 of the probe; the rest: the constraints
+template <int S>
+__global__ __launch_bounds__(Frame<S>::T) void k_constraint_fft(ConstraintArgs c, const cf* probe, cf* phat) {
+  if (blockIdx.x == 0) fft2_body<S, false>(probe, phat, 0, 0);
+  else constraint_apply_body(c, (int)blockIdx.x - 1, (int)gridDim.x - 1);
 }
 
 // sum over the work group of a per-thread float64 value (thread 0 holds it
@@ -1382,38 +1623,23 @@ int grid_for(long long n, int threads, int cap = 4096) {
   return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
-int launch_object_update(cf* obj, const cf* grad, const float* spsum, const float* tilemax, int ntiles,
-                         int Px, int Py, float step, float nmin, hipStream_t stream, int replace = 0) {
-  const long long npix = (long long)Px * Py;
-  const float c1 = (float)(1.0 - (double)nmin), c2 = nmin;
-  hipLaunchKernelGGL(k_object_update, dim3(grid_for(npix, 256)), dim3(256), 0, stream, obj, grad, spsum,
-                     tilemax, ntiles, npix, step, c1, c2, replace);
+ObjectUpdate object_update(cf* obj, float* pot, const cf* grad, const float* spsum, const float* tilemax, int ntiles,
+                           int Px, int Py, float step, float nmin, int replace = 0) {
+  ObjectUpdate u{};
+  u.obj = obj; u.pot = pot; u.grad = grad; u.spsum = spsum; u.tilemax = tilemax; u.ntiles = ntiles;
+  u.npix = (long long)Px * Py; u.step = step; u.c1 = (float)(1.0 - (double)nmin); u.c2 = nmin; u.replace = replace;
+  return u;
+}
+
+// two pixels per thread, and with the probe's work groups beside them
+// (npix / 256, 64 at 128 px) no more than two work groups per CU: every one
+// reads the tile maxima, and a second round of work groups doubled the launch
+// (720^2 pixels with one pixel per thread: 9.8 us against 5 us)
+int object_update_blocks(const ObjectUpdate& u) { return grid_for(u.npix, 2048, 440); }
+
+int launch_object_update(const ObjectUpdate& u, hipStream_t stream) {
+  hipLaunchKernelGGL(k_object_update, dim3(object_update_blocks(u)), dim3(1024), 0, stream, u);
   return check_launch("k_object_update");
-}
-
-int launch_object_update_fft(cf* obj, const cf* grad, const float* spsum, const float* tilemax, int ntiles, int Px,
-                             int Py, float step, float nmin, const cf* probe, cf* phat, int S, hipStream_t stream) {
-  const long long npix = (long long)Px * Py;
-  const float c1 = (float)(1.0 - (double)nmin), c2 = nmin;
-  if (S == 32)
-    hipLaunchKernelGGL(k_object_update_fft<32>, dim3(1 + grid_for(npix, Frame<32>::T)), dim3(Frame<32>::T), 0, stream,
-                       obj, grad, spsum, tilemax, ntiles, npix, step, c1, c2, probe, phat);
-  else if (S == 64)
-    hipLaunchKernelGGL(k_object_update_fft<64>, dim3(1 + grid_for(npix, Frame<64>::T)), dim3(Frame<64>::T), 0, stream,
-                       obj, grad, spsum, tilemax, ntiles, npix, step, c1, c2, probe, phat);
-  else
-    hipLaunchKernelGGL(k_object_update_fft<128>, dim3(1 + grid_for(npix, Frame<128>::T)), dim3(Frame<128>::T), 0,
-                       stream, obj, grad, spsum, tilemax, ntiles, npix, step, c1, c2, probe, phat);
-  return check_launch("k_object_update_fft");
-}
-
-int launch_object_update_potential(float* V, const cf* grad, const float* spsum, const float* tilemax, int ntiles,
-                                   int Px, int Py, float step, float nmin, hipStream_t stream) {
-  const long long npix = (long long)Px * Py;
-  const float c1 = (float)(1.0 - (double)nmin), c2 = nmin;
-  hipLaunchKernelGGL(k_object_update_potential, dim3(grid_for(npix, 256)), dim3(256), 0, stream, V, grad, spsum,
-                     tilemax, ntiles, npix, step, c1, c2);
-  return check_launch("k_object_update_potential");
 }
 
 __host__ __device__ inline int probe_nchunk(int B) { return (B + PROBE_CHUNK - 1) / PROBE_CHUNK; }
@@ -1425,39 +1651,63 @@ size_t probe_ws_bytes(int S, int B) {
          align256((S2 / 256 + 1) * 4);
 }
 
-int launch_probe_apply(cf* probe, double* ws, int S, int B, float step, float nmin, hipStream_t stream,
-                       int replace = 0) {
+ProbeStep probe_step(cf* probe, double* ws, int S, int B, float step, float nmin, int replace = 0) {
   const size_t S2 = (size_t)S * S;
-  char* base = (char*)ws;
-  double* part = ws;
-  cf* gsum = (cf*)(base + align256((size_t)probe_nchunk(B) * S2 * 24));
-  float* osum = (float*)((char*)gsum + align256(S2 * 8));
-  float* bmax = (float*)((char*)osum + align256(S2 * 4));
-  const int npix = (int)S2, nblk = (npix + 255) / 256;
-  hipLaunchKernelGGL(k_probe_reduce, dim3(nblk), dim3(PROBE_REDUCE_THREADS), 0, stream, part, probe_nchunk(B), npix, gsum, osum,
-                     bmax);
-  int rc = check_launch("k_probe_reduce");
-  if (rc) return rc;
-  const float c1 = (float)(1.0 - (double)nmin), c2 = nmin;
-  hipLaunchKernelGGL(k_probe_apply, dim3(nblk), dim3(256), 0, stream, probe, gsum, osum, bmax, nblk, npix, step,
-                     c1, c2, replace);
-  return check_launch("k_probe_apply");
+  ProbeStep q{};
+  q.part = ws; q.nchunk = probe_nchunk(B); q.npix = (int)S2;
+  q.gsum = (cf*)((char*)ws + align256((size_t)q.nchunk * S2 * 24));
+  q.osum = (float*)((char*)q.gsum + align256(S2 * 8));
+  q.bmax = (float*)((char*)q.osum + align256(S2 * 4));
+  q.probe = probe; q.step = step; q.c1 = (float)(1.0 - (double)nmin); q.c2 = nmin; q.replace = replace;
+  return q;
+}
+
+// the probe's chunk sums and, with an object to update, the object step
+int launch_update_reduce(const ProbeStep& q, const ObjectUpdate* u, hipStream_t stream) {
+  const ObjectUpdate none{};
+  hipLaunchKernelGGL(k_update_reduce, dim3(q.npix / 256 + (u ? object_update_blocks(*u) : 0)),
+                     dim3(PROBE_REDUCE_THREADS), 0, stream, q, u ? *u : none);
+  return check_launch("k_update_reduce");
+}
+
+// the probe step after launch_update_reduce; with phat also fft2 of the new
+// probe (S = 32, 64, 128)
+int launch_probe_apply(const ProbeStep& q, int S, cf* phat, hipStream_t stream) {
+  if (!phat) {
+    hipLaunchKernelGGL(k_probe_apply, dim3(q.npix / 256), dim3(256), 0, stream, q);
+    return check_launch("k_probe_apply");
+  }
+  if (S == 32) hipLaunchKernelGGL(k_probe_apply_fft<32>, dim3(1), dim3(Frame<32>::T), 0, stream, q, phat);
+  else if (S == 64) hipLaunchKernelGGL(k_probe_apply_fft<64>, dim3(1), dim3(Frame<64>::T), 0, stream, q, phat);
+  else {
+    const dim3 grid(128 / PROBE_LINES);
+    hipLaunchKernelGGL(k_probe_apply_cols<128>, grid, dim3(256), 0, stream, q, phat);
+    hipLaunchKernelGGL(k_probe_rows<128>, grid, dim3(PROBE_LINES * Frame<128>::N2), 0, stream, phat);
+  }
+  return check_launch("k_probe_apply_fft");
 }
 
 // the scatter of a stage and its probe partial sums
 int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStream_t stream) {
-  const int pix_blocks = (pa.S * pa.S + 255) / 256, nchunk = probe_nchunk(pa.B);
+  const int nchunk = probe_nchunk(pa.B);
   if (!scatter_in_range(g.B, g.S)) {
     int rc = launch_scatter(g, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_probe_partial, dim3(pix_blocks, nchunk), dim3(256), 0, stream, pa);
+    hipLaunchKernelGGL(k_probe_partial, dim3(pa.S * pa.S / (4 * PROBE_PIX), nchunk), dim3(256), 0, stream, pa);
     return check_launch("k_probe_partial");
   }
   const ScatterPlan plan = scatter_plan(g.Px, g.Py);
   const int ns = scatter_blocks(g.Px, g.Py);
+  const int rp = probe_pixels_per_lane(pa.S, nchunk), pix_blocks = pa.S * pa.S / (rp * PROBE_PIX);
   const dim3 grid(ns + pix_blocks * nchunk), blk(256);
-  if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter_probe<1>, grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
-  else hipLaunchKernelGGL(k_scatter_probe<4>, grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  if (plan.rows_per_lane == 1 && rp == 1)
+    hipLaunchKernelGGL((k_scatter_probe<1, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  else if (plan.rows_per_lane == 1)
+    hipLaunchKernelGGL((k_scatter_probe<1, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  else if (rp == 1)
+    hipLaunchKernelGGL((k_scatter_probe<4, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+  else
+    hipLaunchKernelGGL((k_scatter_probe<4, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
   return check_launch("k_scatter_probe");
 }
 
@@ -1466,10 +1716,12 @@ int launch_probe_update(cf* probe, const cf* chi, const cf* obj, int Px, int Py,
                         hipStream_t stream) {
   ProbePartialArgs pa{chi, obj, pos, order, N, B, S, Px, Py, part};
   const int nchunk = probe_nchunk(B);
-  hipLaunchKernelGGL(k_probe_partial, dim3((S * S + 255) / 256, nchunk), dim3(256), 0, stream, pa);
+  hipLaunchKernelGGL(k_probe_partial, dim3(S * S / (4 * PROBE_PIX), nchunk), dim3(256), 0, stream, pa);
   int rc = check_launch("k_probe_partial");
   if (rc) return rc;
-  return launch_probe_apply(probe, part, S, B, step, nmin, stream);
+  const ProbeStep q = probe_step(probe, part, S, B, step, nmin);
+  if ((rc = launch_update_reduce(q, nullptr, stream))) return rc;
+  return launch_probe_apply(q, S, nullptr, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1728,7 +1980,7 @@ __global__ __launch_bounds__(256) void k_lin_right(const cf* __restrict__ T, con
 
 // float64 partial sums of the object (re, im) per block, fixed grid
 constexpr int MEAN_BLOCKS = 256;
-static_assert(MEAN_BLOCKS <= CONSTRAINT_BLOCKS, "mean partials share the constraint partial buffer");
+static_assert(MEAN_BLOCKS <= CONSTRAINT_PARTS, "mean partials share the constraint partial buffer");
 __global__ __launch_bounds__(256) void k_complex_sum_partial(const cf* __restrict__ obj, long long npix,
                                                              double* __restrict__ part) {
   __shared__ double sr[256], si[256];
@@ -1835,32 +2087,58 @@ int launch_object_filters(cf* obj, int Px, int Py, const pty_gd_params& q, void*
   return rc;
 }
 
-int launch_constraints(cf* obj, int Px, int Py, const unsigned char* mask, float shrink, int pure,
-                       double* part, hipStream_t stream) {
-  const long long npix = (long long)Px * Py;
-  if (mask) {
-    hipLaunchKernelGGL(k_constraint_partial, dim3(CONSTRAINT_BLOCKS), dim3(256), 0, stream, obj, mask, npix,
-                       part, (const float*)nullptr);
-    int rc = check_launch("k_constraint_partial");
-    if (rc) return rc;
-  }
-  hipLaunchKernelGGL(k_constraint_apply, dim3(grid_for(npix, 256)), dim3(256), 0, stream, obj, npix, part,
-                     CONSTRAINT_BLOCKS, mask ? 1 : 0, shrink, pure);
+ConstraintArgs constraint_args(cf* obj, float* pot, int Px, int Py, const unsigned char* mask, float shrink, int pure,
+                               int positivity, double* part) {
+  ConstraintArgs c{};
+  c.obj = obj; c.pot = pot; c.mask = mask; c.npix = (long long)Px * Py; c.part = part; c.shrinkage_rad = shrink;
+  c.pure_phase = pure; c.positivity = positivity;
+  return c;
+}
+
+int launch_constraint_apply(const ConstraintArgs& c, hipStream_t stream) {
+  hipLaunchKernelGGL(k_constraint_apply, dim3(grid_for(c.npix, 256)), dim3(256), 0, stream, c);
   return check_launch("k_constraint_apply");
 }
 
-int launch_constraints_potential(float* V, int Px, int Py, const unsigned char* mask, float shrink, int positivity,
-                                 double* part, hipStream_t stream) {
-  const long long npix = (long long)Px * Py;
-  if (mask) {
-    hipLaunchKernelGGL(k_constraint_partial, dim3(CONSTRAINT_BLOCKS), dim3(256), 0, stream, (const cf*)nullptr, mask,
-                       npix, part, (const float*)V);
+int launch_constraints(const ConstraintArgs& c, hipStream_t stream) {
+  if (c.mask) {
+    hipLaunchKernelGGL(k_constraint_partial, dim3(CONSTRAINT_PARTS / 2), dim3(256), 0, stream, c);
     int rc = check_launch("k_constraint_partial");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_constraint_apply_potential, dim3(grid_for(npix, 256)), dim3(256), 0, stream, V, npix, part,
-                     CONSTRAINT_BLOCKS, mask ? 1 : 0, shrink, positivity);
-  return check_launch("k_constraint_apply_potential");
+  return launch_constraint_apply(c, stream);
+}
+
+template <int S>
+void launch_iteration_sums_lds(const ErrorArgs& e, const ConstraintArgs& c, cf* probe, hipStream_t stream) {
+  constexpr int T = Frame<S>::T;
+  const int blocks = 2 + (c.mask ? CONSTRAINT_PARTS / (T / 128) : 0);
+  hipLaunchKernelGGL(k_iteration_sums<S>, dim3(blocks), dim3(T), 0, stream, e, c, probe);
+}
+
+// the error, the constraint's sums and, with a probe (S = 32, 64, 128), its
+// recentring
+int launch_iteration_sums(const ErrorArgs& e, const ConstraintArgs& c, cf* probe, int S, hipStream_t stream) {
+  if (!probe)
+    hipLaunchKernelGGL(k_iteration_sums_only, dim3(1 + (c.mask ? CONSTRAINT_PARTS / 2 : 0)), dim3(256), 0, stream, e, c);
+  else if (S == 32) launch_iteration_sums_lds<32>(e, c, probe, stream);
+  else if (S == 64) launch_iteration_sums_lds<64>(e, c, probe, stream);
+  else launch_iteration_sums_lds<128>(e, c, probe, stream);
+  return check_launch("k_iteration_sums");
+}
+
+template <int S>
+void launch_constraint_fft_lds(const ConstraintArgs& c, const cf* probe, cf* phat, hipStream_t stream) {
+  constexpr int T = Frame<S>::T;
+  hipLaunchKernelGGL(k_constraint_fft<S>, dim3(1 + grid_for(c.npix, T)), dim3(T), 0, stream, c, probe, phat);
+}
+
+// the constraints and fft2 of the probe (S = 32, 64, 128)
+int launch_constraint_fft(const ConstraintArgs& c, const cf* probe, cf* phat, int S, hipStream_t stream) {
+  if (S == 32) launch_constraint_fft_lds<32>(c, probe, phat, stream);
+  else if (S == 64) launch_constraint_fft_lds<64>(c, probe, phat, stream);
+  else launch_constraint_fft_lds<128>(c, probe, phat, stream);
+  return check_launch("k_constraint_fft");
 }
 
 // probe recentring; 256 px frames need `tmp` (one frame) and `shift` (2
@@ -2035,7 +2313,7 @@ WsLayout layout(const pty_problem& p, const pty_gd_params& q, bool positions = f
   L.spsum = o; o = align256(o + npix * 4);
   L.tilemax = o; o = align256(o + (size_t)scatter_num_tiles(p.Px, p.Py) * 4);
   L.ppart = o; o = align256(o + (q.fix_probe ? 0 : probe_ws_bytes(p.S, q.max_batch)));
-  L.cpart = o; o = align256(o + (size_t)CONSTRAINT_BLOCKS * 16);
+  L.cpart = o; o = align256(o + (size_t)CONSTRAINT_PARTS * 16);
   L.run = o; o = align256(o + ((int)B < q.max_batch ? npix * 24 : 0));
   L.far = o; o = align256(o + (positions ? B * S2 * 8 : 0));
   L.total = o;
@@ -2069,10 +2347,10 @@ int validate_problem(const pty_problem* p) {
 // hipGetSymbolAddress, never the array's name.
 // ---------------------------------------------------------------------------
 // SCRATCH_EXTRA: room beyond the documented size for the scatter's tile
-// maxima (scatter_num_tiles is up to eight times the 8 x 64 tiles that
-// fit_stage_to_scratch counts, so that it accepts what it always accepted):
-// 4 bytes per 64 pixels up to SCATTER_SMALL_PIXELS, per 256 beyond, of an
-// object that fits the scratch (under 2 M pixels), 31 KiB at most.
+// maxima and the constraint's partial sums: fit_stage_to_scratch counts 8 x
+// 64 tiles and 256 parts, so that it accepts what it always accepted.  4
+// bytes per 64 pixels up to SCATTER_SMALL_PIXELS, per 256 beyond, of an
+// object that fits the scratch (under 2 M pixels), 31 KiB at most, and 4 KiB.
 constexpr size_t SCRATCH_EXTRA = 64 * 1024;
 static __device__ __align__(256) unsigned char scratch[PTY_NOALLOC_SCRATCH_BYTES + SCRATCH_EXTRA];
 
@@ -2108,7 +2386,7 @@ int fit_stage_to_scratch(const pty_problem& p, pty_gd_params& q) {
   int s = (q.stage > 0 && q.stage < q.max_batch) ? stage_size(q) : q.max_batch;
   size_t need = 0;
   const size_t extra = align256((size_t)scatter_num_tiles(p.Px, p.Py) * 4) -
-                       align256((size_t)gather_num_tiles(p.Px, p.Py) * 4);
+                       align256((size_t)gather_num_tiles(p.Px, p.Py) * 4) + (CONSTRAINT_PARTS - 256) * 16;
   while (true) {
     t.stage = s >= q.max_batch ? 0 : s;
     need = layout(p, t).total - extra;
@@ -2186,10 +2464,13 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
   const int ntiles = scatter_num_tiles(p.Px, p.Py);
   const double norm = (double)(float)(p.mean_intensity * (float)p.N);
   bool phat_valid = false;
-  // complex object with probe update: the object step carries the fft2 of
-  // the updated probe (k_object_update_fft), so phat stays current across
-  // the mini-batches of an iteration
-  const bool fft_with_update = !q.fix_probe && !pot && p.S != 256;
+  // with probe update the probe step carries the fft2 of the updated probe,
+  // so phat stays current across the mini-batches of an iteration; the last
+  // one's probe is recentred or constrained first, and transformed beside
+  // the object constraints or at the start of the next iteration
+  const bool lds_frame = p.S != 256;
+  const bool extra = !q.fix_probe && (q.fix_probe_aperture || q.constrain_probe_amplitude);
+  const bool recentre = !q.fix_probe && q.fix_probe_com;
   for (int it = 0; it < q.num_iter; ++it) {
     const int* order_it = orders + (size_t)it * p.N;
     int start = 0;
@@ -2197,7 +2478,7 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
       const int* ob = order_it + start;
       if (!phat_valid) {
         if ((rc = launch_fft(probe, phat, 1, p.S, false, 0, stream))) return rc;
-        phat_valid = q.fix_probe != 0 || fft_with_update;
+        phat_valid = true;
       }
       int k = 0;
       for (int s0 = 0; s0 < nb; s0 += stage, ++k) {
@@ -2239,47 +2520,44 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
       if (pipe && (rc = hip_check(hipStreamWaitEvent(stream, pipe->scatter_done[(k - 1) & 1], 0),
                                   "hipStreamWaitEvent")))
         return rc;
-      // the probe step first: the object step may carry the probe's fft2
-      if (!q.fix_probe) {
-        if ((rc = launch_probe_apply(probe, ppart, p.S, nb, q.step_size, q.normalization_min, stream))) return rc;
+      const ObjectUpdate u = object_update(obj, V, grad, spsum, tilemax, ntiles, p.Px, p.Py, q.step_size,
+                                           q.normalization_min);
+      if (q.fix_probe) {
+        if ((rc = launch_object_update(u, stream))) return rc;
+      } else {
+        const ProbeStep ps_step = probe_step(probe, ppart, p.S, nb, q.step_size, q.normalization_min);
+        const bool last = start + nb == p.N;
+        phat_valid = lds_frame && !(last && (recentre || extra));
+        if ((rc = launch_update_reduce(ps_step, &u, stream))) return rc;
+        if ((rc = launch_probe_apply(ps_step, p.S, phat_valid ? phat : nullptr, stream))) return rc;
       }
-      if (fft_with_update) {
-        if ((rc = launch_object_update_fft(obj, grad, spsum, tilemax, ntiles, p.Px, p.Py, q.step_size,
-                                           q.normalization_min, probe, phat, p.S, stream)))
-          return rc;
-      } else if (pot) {
-        if ((rc = launch_object_update_potential(V, grad, spsum, tilemax, ntiles, p.Px, p.Py, q.step_size,
-                                                 q.normalization_min, stream)))
-          return rc;
-      } else if ((rc = launch_object_update(obj, grad, spsum, tilemax, ntiles, p.Px, p.Py, q.step_size,
-                                     q.normalization_min, stream)))
-        return rc;
-      if (!q.fix_probe && !fft_with_update) phat_valid = false;
       if (correct) {  // singleslice_ptychography.py:913-926, after the adjoint
         const PosArgs pa = position_args(*pp, ps, far, obj, p.Px, p.Py, p.amplitudes, p.N, ob, nb);
         if ((rc = launch_position_correction(pa, p.S, stream))) return rc;
       }
       start += nb;
     }
-    hipLaunchKernelGGL(k_error_reduce, dim3(1), dim3(1024), 0, stream, err, p.N, norm, errors + it);
-    if ((rc = check_launch("k_error_reduce"))) return rc;
     if (pot) {
       if (q.gaussian_weights && q.gaussian_radius >= 0 &&
           (rc = launch_gaussian_real(V, p.Px, p.Py, q.gaussian_weights, q.gaussian_radius, grad, stream)))
         return rc;
-      if ((rc = launch_constraints_potential(V, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad, q.object_positivity,
-                                             cpart, stream)))
-        return rc;
     } else if ((rc = launch_object_filters(obj, p.Px, p.Py, q, grad, cpart, stream))) {
       return rc;
-    } else if ((rc = launch_constraints(obj, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad, q.pure_phase_object, cpart,
-                                 stream)))
+    }
+    const ErrorArgs ea{err, p.N, norm, errors + it};
+    const ConstraintArgs ca = constraint_args(obj, V, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad,
+                                              q.pure_phase_object, q.object_positivity, cpart);
+    if ((rc = launch_iteration_sums(ea, ca, recentre && lds_frame ? probe : nullptr, p.S, stream))) return rc;
+    if (recentre && lds_frame && !extra && it + 1 < q.num_iter) {
+      if ((rc = launch_constraint_fft(ca, probe, phat, p.S, stream))) return rc;
+      phat_valid = true;
+    } else if ((rc = launch_constraint_apply(ca, stream))) {
       return rc;
-    if (!q.fix_probe && q.fix_probe_com) {
+    }
+    if (recentre && !lds_frame) {
       if ((rc = launch_probe_com(probe, p.S, stream, grad, (float*)cpart))) return rc;
     }
     if (!q.fix_probe && (rc = launch_probe_extra(probe, 1, p.S, q, stream))) return rc;
-    if (!q.fix_probe) phat_valid = false;  // the recentring and constraints moved the probe
     if (correct && pp->center_of_mass) {
       if ((rc = launch_positions_com(pp->positions, p.N, pp->initial_com, stream))) return rc;
     }
@@ -2374,9 +2652,10 @@ int proj_run(const pty_problem* problem, const pty_gd_params* params, const pty_
       }
     }
     valid = 1;
-    hipLaunchKernelGGL(k_error_reduce, dim3(1), dim3(1024), 0, stream, err, p.N, norm, errors + it);
-    if ((rc = check_launch("k_error_reduce"))) return rc;
     if (correct) {
+      // err is overwritten below
+      hipLaunchKernelGGL(k_error_reduce, dim3(1), dim3(1024), 0, stream, err, p.N, norm, errors + it);
+      if ((rc = check_launch("k_error_reduce"))) return rc;
       // the overlap's far field with the object and probe of this iteration's
       // forward pass (singleslice_ptychography.py:913-926 passes `overlap`);
       // the gradient-descent pass forms it (its chi and err are not used)
@@ -2386,22 +2665,32 @@ int proj_run(const pty_problem* problem, const pty_gd_params* params, const pty_
       a.ps_out = ps; a.chi_out = chi; a.err = err; a.fwd_out = far;
       if ((rc = launch_fused(a, p.S, stream))) return rc;
     }
-    if ((rc = launch_object_update(obj, grad, spsum, tilemax, ntiles, p.Px, p.Py, 0.f, q.normalization_min, stream,
-                                   1)))
-      return rc;
-    if (!q.fix_probe) {
-      if ((rc = launch_probe_apply(probe, ppart, p.S, p.N, 0.f, q.normalization_min, stream, 1))) return rc;
+    const ObjectUpdate u = object_update(obj, nullptr, grad, spsum, tilemax, ntiles, p.Px, p.Py, 0.f,
+                                         q.normalization_min, 1);
+    if (q.fix_probe) {
+      if ((rc = launch_object_update(u, stream))) return rc;
+    } else {
+      const ProbeStep ps_step = probe_step(probe, ppart, p.S, p.N, 0.f, q.normalization_min, 1);
+      if ((rc = launch_update_reduce(ps_step, &u, stream))) return rc;
+      if ((rc = launch_probe_apply(ps_step, p.S, nullptr, stream))) return rc;
     }
     if (correct) {  // after the adjoint, with the updated object
       const PosArgs pa = position_args(*pp, ps, far, obj, p.Px, p.Py, p.amplitudes, p.N, order, p.N);
       if ((rc = launch_position_correction(pa, p.S, stream))) return rc;
     }
     if ((rc = launch_object_filters(obj, p.Px, p.Py, q, grad, cpart, stream))) return rc;
-    if ((rc = launch_constraints(obj, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad, q.pure_phase_object, cpart,
-                                 stream)))
-      return rc;
-    if (!q.fix_probe && q.fix_probe_com) {
-      if ((rc = launch_probe_com(probe, p.S, stream))) return rc;
+    const ErrorArgs ea{err, p.N, norm, correct ? nullptr : errors + it};
+    const ConstraintArgs ca = constraint_args(obj, nullptr, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad,
+                                              q.pure_phase_object, 0, cpart);
+    const bool recentre = !q.fix_probe && q.fix_probe_com;
+    const bool extra = !q.fix_probe && (q.fix_probe_aperture || q.constrain_probe_amplitude);
+    if ((rc = launch_iteration_sums(ea, ca, recentre ? probe : nullptr, p.S, stream))) return rc;
+    if (!q.fix_probe && !extra && it + 1 < q.num_iter) {
+      if ((rc = launch_constraint_fft(ca, probe, phat, p.S, stream))) return rc;
+      phat_valid = true;
+    } else {
+      if ((rc = launch_constraint_apply(ca, stream))) return rc;
+      if (!q.fix_probe) phat_valid = false;
     }
     if (!q.fix_probe && (rc = launch_probe_extra(probe, 1, p.S, q, stream))) return rc;
     if (correct && pp->center_of_mass) {
@@ -2434,7 +2723,7 @@ MixedLayout mixed_layout(const pty_problem& p, const pty_gd_params& q, int K, bo
   L.bmax = o; o = align256(o + MIXED_BLOCKS * 4);
   L.pstride = q.fix_probe ? 0 : align256(probe_ws_bytes(p.S, q.max_batch));
   L.ppart = o; o = align256(o + K * L.pstride);
-  L.cpart = o; o = align256(o + (size_t)CONSTRAINT_BLOCKS * 16);
+  L.cpart = o; o = align256(o + (size_t)CONSTRAINT_PARTS * 16);
   L.shift = o; o = align256(o + 8);
   L.acc = o; o = align256(o + (positions ? 3 * B * S2 * 4 : 0));
   L.all = o;
@@ -2525,9 +2814,10 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
       if ((rc = check_launch("k_mixed_object_update"))) return rc;
       if (!q.fix_probe) {
         for (int k = 0; k < K; ++k) {
-          if ((rc = launch_probe_apply(probe + (size_t)k * S2, (double*)(ws + L.ppart + k * L.pstride), p.S, nb,
-                                       q.step_size, q.normalization_min, stream)))
-            return rc;
+          const ProbeStep step = probe_step(probe + (size_t)k * S2, (double*)(ws + L.ppart + k * L.pstride), p.S, nb,
+                                            q.step_size, q.normalization_min);
+          if ((rc = launch_update_reduce(step, nullptr, stream))) return rc;
+          if ((rc = launch_probe_apply(step, p.S, nullptr, stream))) return rc;
         }
       }
       if (pp) {  // position correction with the updated object (mixedstate_ptychography.py:942-956)
@@ -2553,12 +2843,12 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
       }
       start += nb;
     }
-    hipLaunchKernelGGL(k_error_reduce, dim3(1), dim3(1024), 0, stream, err, p.N, norm, errors + it);
-    if ((rc = check_launch("k_error_reduce"))) return rc;
     if ((rc = launch_object_filters(obj, p.Px, p.Py, q, grad, cpart, stream))) return rc;
-    if ((rc = launch_constraints(obj, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad, q.pure_phase_object, cpart,
-                                 stream)))
-      return rc;
+    const ErrorArgs ea{err, p.N, norm, errors + it};
+    const ConstraintArgs ca = constraint_args(obj, nullptr, p.Px, p.Py, p.fov_mask_inverse, q.shrinkage_rad,
+                                              q.pure_phase_object, 0, cpart);
+    if ((rc = launch_iteration_sums(ea, ca, nullptr, p.S, stream))) return rc;
+    if ((rc = launch_constraint_apply(ca, stream))) return rc;
     if (!q.fix_probe && q.fix_probe_com) {
       if ((rc = launch_probe_com_modes(probe, K, p.S, (float*)(ws + L.shift), stream))) return rc;
     }
@@ -2642,8 +2932,9 @@ int pty_object_update(void* object, const void* grad, const float* spsum, const 
                       int Py, float step_size, float normalization_min, pty_stream_t stream) {
   if (!object || !grad || !spsum || !tilemax || ntiles <= 0 || Px <= 0 || Py <= 0)
     return fail(PTY_E_ARG, "bad object update arguments");
-  return launch_object_update((cf*)object, (const cf*)grad, spsum, tilemax, ntiles, Px, Py, step_size,
-                              normalization_min, st(stream));
+  return launch_object_update(object_update((cf*)object, nullptr, (const cf*)grad, spsum, tilemax, ntiles, Px, Py,
+                                            step_size, normalization_min),
+                              st(stream));
 }
 
 size_t pty_probe_partials_bytes(int S, int B) { return probe_ws_bytes(S, B); }
@@ -2661,12 +2952,13 @@ int pty_probe_update(void* probe, const void* chi, const void* object, int Px, i
                              step_size, normalization_min, (double*)partials, st(stream));
 }
 
-size_t pty_constraint_partials_bytes(void) { return (size_t)CONSTRAINT_BLOCKS * 16; }
+size_t pty_constraint_partials_bytes(void) { return (size_t)CONSTRAINT_PARTS * 16; }
 
 int pty_object_constraints(void* object, int Px, int Py, const unsigned char* mask, float shrinkage_rad,
                            int pure_phase_object, void* partials, pty_stream_t stream) {
   if (!object || Px <= 0 || Py <= 0 || (mask && !partials)) return fail(PTY_E_ARG, "bad constraint arguments");
-  return launch_constraints((cf*)object, Px, Py, mask, shrinkage_rad, pure_phase_object, (double*)partials,
+  return launch_constraints(constraint_args((cf*)object, nullptr, Px, Py, mask, shrinkage_rad, pure_phase_object, 0,
+                                            (double*)partials),
                             st(stream));
 }
 
