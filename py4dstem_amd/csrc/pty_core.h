@@ -436,7 +436,8 @@ struct FusedArgs {
   int N, B, Px, Py;
   int b0;                  // first batch slot handled by this launch
   cf* ps_out;              // [B][S][S] shifted probe P_shift      (natural)
-  cf* chi_out;             // [B][S][S] chi = ifft2(A e^{i angle F} - F) (natural)
+  cf* chi_out;             // [B][S][S] chi = ifft2(A e^{i angle F} - F) (natural); null (32-128 px
+                           // gradient-descent pass): the pass ends with the errors
   double* err;             // [B] sum (A - |F|)^2 per position
   cf* fwd_out;             // optional [B][N1][T] far field F, element j of thread t of the
                            // row pass at [j][t] (coalesced; see far_index), or null
@@ -461,6 +462,9 @@ struct FusedArgs {
   // 1522-1523): float32 V [Px][Py]; the patch is exp(i V).  Read by the
   // gradient-descent pass instantiated for it, in place of `object`
   const float* object_pot;
+  // 256 px frames: room for 16 partial errors per slot of the launch (from
+  // slot b0), or null
+  double* err_part;
 };
 
 // exp(i v) as NumPy's complex64 exp(1j * v): (cos v, sin v)
@@ -966,6 +970,10 @@ PTY_HD void fused_position(Run& run, const FusedArgs& a, int b) {
   run.phase([&](int tid, Regs& r, auto lds, const cf* tw) {
     K::template p_project<decltype(lds), false, MASK>(tid, a, b, r, lds, tw);
   });
+  if (!a.chi_out) {  // the error alone (the differentiable loss's forward pass)
+    run.reduce_err(b);
+    return;
+  }
   run.wave_barrier();
   run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::template p_rowA<true>(tid, r, lds, tw); });
   run.barrier();

@@ -2494,6 +2494,9 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
         a.order = ob + s0; a.N = p.N; a.B = ns; a.Px = p.Px; a.Py = p.Py; a.b0 = 0;
         a.ps_out = ps_k; a.chi_out = chi_k; a.err = err + start + s0; a.fwd_out = far;
         a.fmask = p.fourier_mask;
+        // the scatter's object sums are not live during the fused pass of an
+        // unpipelined run: room for the partial errors of 256 px frames
+        a.err_part = !pipe && (long long)ns * 16 <= (long long)p.Px * p.Py ? (double*)grad : nullptr;
         if ((rc = launch_fused(a, p.S, stream))) return rc;
         if (pipe && ((rc = hip_check(hipEventRecord(pipe->fused_done[k & 1], stream), "hipEventRecord")) ||
                      (rc = hip_check(hipStreamWaitEvent(gs, pipe->fused_done[k & 1], 0), "hipStreamWaitEvent"))))
@@ -3075,7 +3078,10 @@ int pty_loss_gradients(const void* object, const void* probe, int Px, int Py, co
     FusedArgs a{};
     a.probe_hat = phat; a.object = (const cf*)object; a.positions = positions; a.amps = amplitudes;
     a.order = order + start; a.N = N; a.B = nb; a.Px = Px; a.Py = Py; a.b0 = 0;
-    a.ps_out = ps; a.chi_out = chi; a.err = err + start; a.fwd_out = nullptr;
+    // without a gradient to form, the errors alone: no stores of P_shift and
+    // chi and no third transform
+    const bool adjoint = grad_object || grad_probe;
+    a.ps_out = grad_object ? ps : nullptr; a.chi_out = adjoint ? chi : nullptr; a.err = err + start; a.fwd_out = nullptr;
     if ((rc = launch_fused(a, S, stream))) return rc;
     if (grad_object) {
       GatherArgs g{};
