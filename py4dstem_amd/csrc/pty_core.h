@@ -802,7 +802,7 @@ template <int S> struct Fused {
   // ---- mixed state (ptychographic_methods.py:2696-2805) -------------------
 
   // row pass B completes F_k; F_k to the staging buffer; sum_k |F_k|^2 in
-  // r.amp (float32, modes in order, |F| as the reference's abs then square)
+  // r.amp (float32, modes in order)
   template <class L> static PTY_HD void p_mixed_far(int tid, const FusedArgs& a, int b, int k,
                                                     Regs& r, L lds, const cf* tw) {
 #if defined(__clang__)
@@ -818,8 +818,7 @@ template <int S> struct Fused {
     for (int j = 0; j < N1; ++j) {
       if (fm) r.v[j] = cscale(r.v[j], fm[j]);
       far[(size_t)j * T] = r.v[j];
-      const float m = hypot_f(r.v[j].x, r.v[j].y);
-      r.amp[j] = (k == 0 ? 0.f : r.amp[j]) + m * m;
+      r.amp[j] = (k == 0 ? 0.f : r.amp[j]) + cabs2(r.v[j]);
     }
   }
 
@@ -837,8 +836,7 @@ template <int S> struct Fused {
       const float far = sqrt_rn(r.amp[j]);
       const float d = amp - far;
       acc += (double)(d * d);
-      // float32 quotient, correctly rounded through float64 (53 >= 2 * 24 + 2)
-      r.amp[j] = far == 0.f ? 0.f : (float)((double)amp / (double)far);
+      r.amp[j] = far == 0.f ? 0.f : amp / far;
     }
     r.err += acc;
   }

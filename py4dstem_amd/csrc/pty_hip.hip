@@ -635,47 +635,6 @@ __global__ __launch_bounds__(1024) void k_object_update(ObjectUpdate u) {
   object_update_body(u, (int)blockIdx.x, (int)gridDim.x);
 }
 
-// mixed state (ptychographic_methods.py:2945-2975): the mode overlaps summed
-// in float32, modes in order, with a per-block maximum
-__global__ __launch_bounds__(256) void k_mixed_overlap(const float* __restrict__ spsum, int K, long long npix,
-                                                       float* __restrict__ total, float* __restrict__ bmax) {
-  __shared__ float sh[16];
-  float m = 0.f;
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    float s = spsum[p];
-    for (int k = 1; k < K; ++k) s = s + spsum[(size_t)k * npix + p];
-    total[p] = s;
-    m = fmaxf(m, s);
-  }
-  m = group_max(m, sh);
-  if (threadIdx.x == 0) bmax[blockIdx.x] = m;
-}
-
-// object += (sum_k step * grad_k) * norm(total), the reference's float32 order
-__global__ __launch_bounds__(256) void k_mixed_object_update(cf* __restrict__ obj, const cf* __restrict__ grad,
-                                                             int K, const float* __restrict__ total,
-                                                             const float* __restrict__ bmax, int nblk,
-                                                             long long npix, float step, float c1, float c2) {
-#pragma clang fp contract(off)
-  __shared__ float sh[16];
-  float m = 0.f;
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x) m = fmaxf(m, bmax[i]);
-  m = group_max(m, sh);
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    float ux = 0.f, uy = 0.f;
-    for (int k = 0; k < K; ++k) {
-      const cf g = grad[(size_t)k * npix + p];
-      ux = ux + step * g.x;
-      uy = uy + step * g.y;
-    }
-    const float n = overlap_norm(total[p], m, c1, c2);
-    const cf o = obj[p];
-    obj[p] = mkcf(o.x + ux * n, o.y + uy * n);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // probe update: partial sums over chunks of the batch, then one work group
 // ---------------------------------------------------------------------------
@@ -817,6 +776,12 @@ __device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, in
   }
 }
 
+// what lies between one probe mode's arrays and the next one's
+struct ModeStride {
+  size_t frames, pixels, tiles;  // elements of the staged frames, object pixels, tile maxima
+  size_t part, probe;            // bytes of the probe partials, elements of the probe
+};
+
 __global__ __launch_bounds__(256) void k_probe_partial(ProbePartialArgs a) {
   __shared__ ProbeShared<4> sh;
   probe_partial_body<4>(a, blockIdx.x, blockIdx.y, sh);
@@ -827,12 +792,22 @@ __global__ __launch_bounds__(256) void k_probe_partial(ProbePartialArgs a) {
 // fused pass's staged terms
 template <int R, int RP>
 __global__ __launch_bounds__(256) void k_scatter_probe(GatherArgs g, ScatterPlan plan, int nscatter,
-                                                       ProbePartialArgs pa, int pix_blocks) {
+                                                       ProbePartialArgs pa, int pix_blocks, ModeStride m) {
   __shared__ union {
     ScatterShared<R> scatter;
     ProbeShared<RP> probe;
   } sh;
   const int b = (int)blockIdx.x;
+  if (gridDim.y > 1) {
+    const size_t k = blockIdx.y;
+    g.ps += k * m.frames;
+    g.chi += k * m.frames;
+    g.grad += k * m.pixels;
+    g.spsum += k * m.pixels;
+    g.tilemax += k * m.tiles;
+    pa.chi += k * m.frames;
+    pa.part = (double*)((char*)pa.part + k * m.part);
+  }
   if (b < nscatter) scatter_body<R>(g, plan, b, sh.scatter);
   else probe_partial_body<RP>(pa, (b - nscatter) % pix_blocks, (b - nscatter) / pix_blocks, sh.probe);
 }
@@ -901,6 +876,16 @@ struct ProbeStep {
   int replace;
 };
 
+// mode k's probe step
+__device__ __forceinline__ ProbeStep mode_step(ProbeStep q, const ModeStride& m, int k) {
+  q.part = (const double*)((const char*)q.part + k * m.part);
+  q.gsum = (cf*)((char*)q.gsum + k * m.part);
+  q.osum = (float*)((char*)q.osum + k * m.part);
+  q.bmax = (float*)((char*)q.bmax + k * m.part);
+  q.probe += k * m.probe;
+  return q;
+}
+
 // the probe's chunk sums (work groups [0, npix / 256)) and the object step
 // (the rest) in one launch: both only read the scatter's and the probe
 // partials' results
@@ -945,6 +930,81 @@ __device__ __forceinline__ void probe_apply_body(const ProbeStep& q, int blk) {
 }
 
 __global__ __launch_bounds__(256) void k_probe_apply(ProbeStep q) { probe_apply_body(q, blockIdx.x); }
+
+// mixed state (ptychographic_methods.py:2945-2975).  Two launches for all
+// modes: the probes' chunk sums beside the mode overlaps summed in float32,
+// modes in order, with a per-block maximum; then the probe steps beside the
+// object step object += (sum_k step * grad_k) * norm(total), the reference's
+// float32 order.
+// Each of these launches works on 16 K pixels to 86 K pixels a mode and took
+// its 4.6 us whatever its size, so one per mode left the chip idle: with three
+// modes at 128 px the eight of a batch took 38 us and take 10.5 us, the three
+// scatters 120 us and 101 us.
+struct MixedUpdate {
+  cf* obj;
+  const cf* grad;      // [K][npix]
+  const float* spsum;  // [K][npix]
+  float* total;        // [npix]
+  float* bmax;         // [nblk]
+  int K, nblk;
+  long long npix;
+  float step, c1, c2;
+};
+
+__device__ __forceinline__ void mixed_overlap_body(const MixedUpdate& u, int blk) {
+  __shared__ float red[16];
+  float m = 0.f;
+  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < u.npix; p += (long long)u.nblk * blockDim.x) {
+    float s = u.spsum[p];
+    for (int k = 1; k < u.K; ++k) s = s + u.spsum[(size_t)k * u.npix + p];
+    u.total[p] = s;
+    m = fmaxf(m, s);
+  }
+  m = group_max(m, red);
+  if (threadIdx.x == 0) u.bmax[blk] = m;
+}
+
+__device__ __forceinline__ void mixed_object_body(const MixedUpdate& u, int blk, int nblk) {
+#pragma clang fp contract(off)
+  __shared__ float red[16];
+  float m = 0.f;
+  for (int i = threadIdx.x; i < u.nblk; i += blockDim.x) m = fmaxf(m, u.bmax[i]);
+  m = group_max(m, red);
+  for (long long p = (long long)blk * blockDim.x + threadIdx.x; p < u.npix; p += (long long)nblk * blockDim.x) {
+    float ux = 0.f, uy = 0.f;
+    for (int k = 0; k < u.K; ++k) {
+      const cf g = u.grad[(size_t)k * u.npix + p];
+      ux = ux + u.step * g.x;
+      uy = uy + u.step * g.y;
+    }
+    const float n = overlap_norm(u.total[p], m, u.c1, u.c2);
+    const cf o = u.obj[p];
+    u.obj[p] = mkcf(o.x + ux * n, o.y + uy * n);
+  }
+}
+
+// work groups [0, K npix / 256): the probes; the rest: the object
+__global__ __launch_bounds__(PROBE_REDUCE_THREADS) void k_mixed_reduce(ProbeStep q, ModeStride m, int nred,
+                                                                      MixedUpdate u) {
+  const int b = (int)blockIdx.x;
+  if (b < nred) {
+    const int per = q.npix / 256;
+    q = mode_step(q, m, b / per);
+    probe_reduce_body(q.part, q.nchunk, q.npix, q.gsum, q.osum, q.bmax, b % per);
+  } else {
+    mixed_overlap_body(u, b - nred);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_mixed_apply(ProbeStep q, ModeStride m, int napply, MixedUpdate u) {
+  const int b = (int)blockIdx.x;
+  if (b < napply) {
+    const int per = q.npix / 256;
+    probe_apply_body(mode_step(q, m, b / per), b % per);
+  } else {
+    mixed_object_body(u, b - napply, (int)gridDim.x - napply);
+  }
+}
 
 // The probe step and fft2 of the new probe (kernel layout) for the next
 // mini-batch, frames of 32 and 64 px: one work group, the updated pixels go
@@ -1302,12 +1362,13 @@ __global__ __launch_bounds__(Frame<S>::T) void k_probe_shift_modes(cf* __restric
   using K = Fused<S>;
   __shared__ cf lds_mem[F::LDS_WORDS];
   __shared__ cf tw[Fused<S>::TW_WORDS];
+  __shared__ cf ramp[2 * S];
   const int tid = threadIdx.x;
   K::twiddles(tid, LdsPtr{tw}, Frame<S>::T);
   LdsPtr lds{lds_mem};
   typename K::Regs r;
   cf* pk = probe + (size_t)blockIdx.x * S * S;
-  const float s0 = shift[0], s1 = shift[1];
+  for (int k = tid; k < 2 * S; k += F::T) ramp[k] = K::ramp1(k % S, shift[k / S]);
   const int cc = F::col_line(tid), n2 = F::col_q(tid);
 #pragma unroll
   for (int m = 0; m < F::N1; ++m) r.v[m] = pk[(n2 + F::N2 * m) * S + cc];
@@ -1325,10 +1386,10 @@ __global__ __launch_bounds__(Frame<S>::T) void k_probe_shift_modes(cf* __restric
 #pragma unroll
     for (int j = 0; j < F::N1; ++j) r.v[j] = lds.ld(F::at(rr, F::N1 * t + j));
     Pass<S>::template B<false>(t, r.v, tw);
-    const cf ex = K::ramp1(F::kidx(rr), s0);
+    const cf ex = ramp[F::kidx(rr)];
 #pragma unroll
     for (int j = 0; j < F::N1; ++j) {
-      const cf e = cmul(ex, K::ramp1(F::kidx(F::N1 * t + j), s1));
+      const cf e = cmul(ex, ramp[S + F::kidx(F::N1 * t + j)]);
       r.v[j] = cmul(r.v[j], e);
     }
     Pass<S>::template B<true>(t, r.v, tw);
@@ -1687,27 +1748,36 @@ int launch_probe_apply(const ProbeStep& q, int S, cf* phat, hipStream_t stream) 
   return check_launch("k_probe_apply_fft");
 }
 
-// the scatter of a stage and its probe partial sums
-int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStream_t stream) {
+// the scatter of a stage and its probe partial sums, of K probe modes
+int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStream_t stream, int K = 1,
+                         const ModeStride& m = ModeStride{}) {
   const int nchunk = probe_nchunk(pa.B);
   if (!scatter_in_range(g.B, g.S)) {
-    int rc = launch_scatter(g, stream);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_probe_partial, dim3(pa.S * pa.S / (4 * PROBE_PIX), nchunk), dim3(256), 0, stream, pa);
-    return check_launch("k_probe_partial");
+    for (int k = 0; k < K; ++k) {
+      GatherArgs gk = g;
+      gk.ps += k * m.frames; gk.chi += k * m.frames; gk.grad += k * m.pixels; gk.spsum += k * m.pixels;
+      gk.tilemax += k * m.tiles;
+      ProbePartialArgs pk = pa;
+      pk.chi += k * m.frames; pk.part = (double*)((char*)pa.part + k * m.part);
+      int rc = launch_scatter(gk, stream);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_probe_partial, dim3(pa.S * pa.S / (4 * PROBE_PIX), nchunk), dim3(256), 0, stream, pk);
+      if ((rc = check_launch("k_probe_partial"))) return rc;
+    }
+    return PTY_OK;
   }
   const ScatterPlan plan = scatter_plan(g.Px, g.Py);
   const int ns = scatter_blocks(g.Px, g.Py);
   const int rp = probe_pixels_per_lane(pa.S, nchunk), pix_blocks = pa.S * pa.S / (rp * PROBE_PIX);
-  const dim3 grid(ns + pix_blocks * nchunk), blk(256);
+  const dim3 grid(ns + pix_blocks * nchunk, K), blk(256);
   if (plan.rows_per_lane == 1 && rp == 1)
-    hipLaunchKernelGGL((k_scatter_probe<1, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+    hipLaunchKernelGGL((k_scatter_probe<1, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks, m);
   else if (plan.rows_per_lane == 1)
-    hipLaunchKernelGGL((k_scatter_probe<1, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+    hipLaunchKernelGGL((k_scatter_probe<1, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks, m);
   else if (rp == 1)
-    hipLaunchKernelGGL((k_scatter_probe<4, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+    hipLaunchKernelGGL((k_scatter_probe<4, 1>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks, m);
   else
-    hipLaunchKernelGGL((k_scatter_probe<4, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks);
+    hipLaunchKernelGGL((k_scatter_probe<4, 4>), grid, blk, 0, stream, g, plan, ns, pa, pix_blocks, m);
   return check_launch("k_scatter_probe");
 }
 
@@ -2775,7 +2845,7 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
   const size_t S2 = (size_t)p.S * p.S;
   const long long npix = (long long)p.Px * p.Py;
   const int ntiles = scatter_num_tiles(p.Px, p.Py);
-  const int nblk = grid_for(npix, 256, MIXED_BLOCKS);
+  const int nblk = grid_for(npix, PROBE_REDUCE_THREADS, 256);  // at most MIXED_BLOCKS
   const std::vector<int> batches = subdivide(p.N, q.max_batch);
   const double norm = (double)(float)(p.mean_intensity * (float)p.N);
   const float c1 = (float)(1.0 - (double)q.normalization_min), c2 = q.normalization_min;
@@ -2795,34 +2865,30 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
       a.ps_out = ps; a.chi_out = chi; a.err = err + start; a.fwd_out = far; a.K = K;
       a.fmask = p.fourier_mask;
       if ((rc = launch_mixed(a, p.S, stream))) return rc;
-      for (int k = 0; k < K; ++k) {
-        const cf* ps_k = ps + (size_t)k * nb * S2;
-        const cf* chi_k = chi + (size_t)k * nb * S2;
-        GatherArgs g{};
-        g.ps = ps_k; g.chi = chi_k; g.positions = p.positions; g.order = ob; g.N = p.N; g.B = nb; g.S = p.S;
-        g.Px = p.Px; g.Py = p.Py; g.tiles_y = gather_tiles_y(p.Py); g.grad = grad + (size_t)k * npix;
-        g.spsum = spsum + (size_t)k * npix; g.tilemax = tilemax + (size_t)k * ntiles;
-        if (q.fix_probe) {
-          if ((rc = launch_scatter(g, stream))) return rc;
-        } else {  // the mode's scatter and probe partial sums in one launch
-          ProbePartialArgs pa{chi_k, obj, p.positions, ob, p.N, nb, p.S, p.Px, p.Py,
-                              (double*)(ws + L.ppart + k * L.pstride)};
-          if ((rc = launch_scatter_probe(g, pa, stream))) return rc;
-        }
-      }
-      hipLaunchKernelGGL(k_mixed_overlap, dim3(nblk), dim3(256), 0, stream, spsum, K, npix, total, bmax);
-      if ((rc = check_launch("k_mixed_overlap"))) return rc;
-      hipLaunchKernelGGL(k_mixed_object_update, dim3(grid_for(npix, 256)), dim3(256), 0, stream, obj, grad, K,
-                         total, bmax, nblk, npix, q.step_size, c1, c2);
-      if ((rc = check_launch("k_mixed_object_update"))) return rc;
-      if (!q.fix_probe) {
+      const ModeStride ms{(size_t)nb * S2, (size_t)npix, (size_t)ntiles, L.pstride, S2};
+      GatherArgs g{};
+      g.ps = ps; g.chi = chi; g.positions = p.positions; g.order = ob; g.N = p.N; g.B = nb; g.S = p.S;
+      g.Px = p.Px; g.Py = p.Py; g.tiles_y = gather_tiles_y(p.Py); g.grad = grad; g.spsum = spsum; g.tilemax = tilemax;
+      ProbeStep step{};
+      if (q.fix_probe) {
         for (int k = 0; k < K; ++k) {
-          const ProbeStep step = probe_step(probe + (size_t)k * S2, (double*)(ws + L.ppart + k * L.pstride), p.S, nb,
-                                            q.step_size, q.normalization_min);
-          if ((rc = launch_update_reduce(step, nullptr, stream))) return rc;
-          if ((rc = launch_probe_apply(step, p.S, nullptr, stream))) return rc;
+          GatherArgs gk = g;
+          gk.ps += k * ms.frames; gk.chi += k * ms.frames; gk.grad += k * ms.pixels; gk.spsum += k * ms.pixels;
+          gk.tilemax += k * ms.tiles;
+          if ((rc = launch_scatter(gk, stream))) return rc;
         }
+      } else {  // every mode's scatter and probe partial sums in one launch
+        const ProbePartialArgs pa{chi, obj, p.positions, ob, p.N, nb, p.S, p.Px, p.Py, (double*)(ws + L.ppart)};
+        if ((rc = launch_scatter_probe(g, pa, stream, K, ms))) return rc;
+        step = probe_step(probe, (double*)(ws + L.ppart), p.S, nb, q.step_size, q.normalization_min);
       }
+      const MixedUpdate mu{obj, grad, spsum, total, bmax, K, nblk, npix, q.step_size, c1, c2};
+      const int probes = q.fix_probe ? 0 : K * (int)S2 / 256;
+      hipLaunchKernelGGL(k_mixed_reduce, dim3(probes + nblk), dim3(PROBE_REDUCE_THREADS), 0, stream, step, ms, probes,
+                         mu);
+      if ((rc = check_launch("k_mixed_reduce"))) return rc;
+      hipLaunchKernelGGL(k_mixed_apply, dim3(probes + grid_for(npix, 256)), dim3(256), 0, stream, step, ms, probes, mu);
+      if ((rc = check_launch("k_mixed_apply"))) return rc;
       if (pp) {  // position correction with the updated object (mixedstate_ptychography.py:942-956)
         PosArgs base = position_args(*pp, ps, far, obj, p.Px, p.Py, p.amplitudes, p.N, ob, nb);
         base.far_modes = K;
