@@ -1900,8 +1900,7 @@ int launch_gaussian_real(float* V, int Px, int Py, const double* w, int r, void*
 // O - mean(O), fft2, times env(|q|) on the fftfreq grid, ifft2, + mean.  The
 // object is any size, so each 2-D transform is two complex products with the
 // DFT matrices (rows, then columns), W[a][b] = exp(-+2 pi i ((a b) mod n) / n)
-// generated in float64 while the tiles are loaded; float32 products, float32
-// accumulation over n terms.
+// generated in float64; float32 products, float32 accumulation over n terms.
 // ---------------------------------------------------------------------------
 constexpr int DFT_T = 32;  // output tile DFT_T x DFT_T, k-step DFT_T
 
@@ -1912,14 +1911,162 @@ __device__ __forceinline__ cf dft_twiddle(int a, int b, int n, int inverse) {
   return mkcf((float)c, (float)s);
 }
 
+// What happens to a value beside the products: the object's mean goes off
+// before the first one, the envelope (with the inverse transform's 1 / (Px
+// Py)) on after the second, the mean back on after the last.
+struct DftArgs {
+  const cf* X;
+  cf* Y;
+  int M, N, inverse;
+  int sub_mean, add_mean, envelope;
+  const double* part;  // [MEAN_BLOCKS][2] partial sums of the object
+  double dx, dy, q_lowpass, q_highpass, order;
+};
+
+constexpr int MEAN_BLOCKS = 256;
+static_assert(MEAN_BLOCKS <= CONSTRAINT_PARTS, "mean partials share the constraint partial buffer");
+
+// mean of the object from its partial sums, by the first wave (four per lane,
+// then a butterfly); every thread returns it
+__device__ __forceinline__ cf mean_from_partials(const double* part, double npix) {
+  __shared__ cf mean_sh;
+  if (threadIdx.x < 64) {
+    double a = 0.0, b = 0.0;
+#pragma unroll
+    for (int k = 0; k < MEAN_BLOCKS / 64; ++k) {
+      a += part[2 * (64 * k + threadIdx.x)];
+      b += part[2 * (64 * k + threadIdx.x) + 1];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      a += __shfl_xor(a, off);
+      b += __shfl_xor(b, off);
+    }
+    if (threadIdx.x == 0) mean_sh = mkcf((float)(a / npix), (float)(b / npix));
+  }
+  __syncthreads();
+  return mean_sh;
+}
+
+// env(|q|) / (Px Py) at spectral pixel (x, y), in float64 as the reference
+// evaluates it
+__device__ __forceinline__ double butterworth_env(const DftArgs& a, int x, int y) {
+  const double vx = 1.0 / (a.M * a.dx), vy = 1.0 / (a.N * a.dy);
+  const int kx = x < (a.M - 1) / 2 + 1 ? x : x - a.M;  // numpy fftfreq order
+  const int ky = y < (a.N - 1) / 2 + 1 ? y : y - a.N;
+  const double qx = kx * vx, qy = ky * vy;
+  const double qr = sqrt(qx * qx + qy * qy);
+  double env = 1.0;
+  if (a.q_highpass != 0.0) env *= 1.0 - 1.0 / (1.0 + pow(qr / a.q_highpass, 2.0 * a.order));
+  if (a.q_lowpass != 0.0) env *= 1.0 / (1.0 + pow(qr / a.q_lowpass, 2.0 * a.order));
+  return env * (1.0 / ((double)a.M * (double)a.N));
+}
+
+__device__ __forceinline__ cf dft_epilogue(const DftArgs& a, cf v, int x, int y, cf mean) {
+  if (a.envelope) {
+    const double f = butterworth_env(a, x, y);
+    v = mkcf((float)((double)v.x * f), (float)((double)v.y * f));
+  }
+  return a.add_mean ? mkcf(v.x + mean.x, v.y + mean.y) : v;
+}
+
 // LEFT:  Y[i][j] = sum_k W_M[i][k] X[k][j]   (transform along axis 0)
 // RIGHT: Y[i][j] = sum_k X[i][k] W_N[k][j]   (transform along axis 1)
+// on v_mfma_f32_16x16x4_f32 (float32 products and sums): a work group makes a
+// 16 x 16 tile, its four waves a quarter of the sum each.  The n roots of
+// unity are tabulated in LDS once per work group (float64 sincospi rounded to
+// float32) and stepped through by index: k i mod n advances by i, so no
+// product, division or trigonometry is left in the loop.  At 284 x 272 pixels
+// a product took 48 us on 32 x 32 tiles with a sincospi per tile element
+// (81 work groups), and takes 8 to 10 us here.
+constexpr int DFT_MAX = 8192;  // roots that fit 64 KiB of LDS
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <bool LEFT> __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
+  extern __shared__ cf root[];  // [n]
+  __shared__ cf partial[3][256];
+  const int n = LEFT ? a.M : a.N;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int m = tid; m < n; m += 256) {
+    double s, c;
+    sincospi((a.inverse ? 2.0 : -2.0) * (double)m / (double)n, &s, &c);
+    root[m] = mkcf((float)c, (float)s);
+  }
+  const cf mean = a.sub_mean || a.add_mean ? mean_from_partials(a.part, (double)((long long)a.M * a.N)) : mkcf(0.f, 0.f);
+  const cf sub = a.sub_mean ? mean : mkcf(0.f, 0.f);
+  __syncthreads();
+  const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
+  const int line = lane & 15, g = lane >> 4;
+  // lane (line, g) of step t supplies W[w][k] and X at k = k0 + 4 g + t
+  const int w = (LEFT ? i0 : j0) + line;   // row of W (LEFT), column of W (RIGHT)
+  const int x = (LEFT ? j0 : i0) + line;   // column of X, row of X
+  const bool wok = w < n, xok = x < (LEFT ? a.N : a.M);
+  // this wave's part of the sum, in runs of 16
+  const int runs = (n + 15) / 16, r0 = runs * wave / 4, r1 = runs * (wave + 1) / 4;
+  const int ws = wok ? w : 0;
+  int idx = (int)((long long)ws * (16 * r0 + 4 * g) % n);  // w k mod n
+  const int jump = (int)((long long)ws * 13 % n);          // from k0 + 4 g + 3 to the next run
+  const size_t stride = LEFT ? (size_t)a.N : 1;
+  const cf* X = a.X + (LEFT ? (size_t)(xok ? x : 0) : (size_t)(xok ? x : 0) * a.N);
+  f32x4 cr = {0.f, 0.f, 0.f, 0.f}, ci = {0.f, 0.f, 0.f, 0.f};
+  cf nx[4];
+  const auto fetch = [&](int r) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int k = 16 * r + 4 * g + t;
+      nx[t] = X[(size_t)(k < n ? k : 0) * stride];
+    }
+  };
+  if (r0 < r1) fetch(r0);
+  for (int r = r0; r < r1; ++r) {
+    cf xv[4], wv[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool ok = 16 * r + 4 * g + t < n;
+      xv[t] = ok && xok ? csub(nx[t], sub) : mkcf(0.f, 0.f);
+      wv[t] = ok && wok ? root[idx] : mkcf(0.f, 0.f);
+      idx += t < 3 ? ws : jump;
+      idx -= idx >= n ? n : 0;
+    }
+    if (r + 1 < r1) fetch(r + 1);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const cf A = LEFT ? wv[t] : xv[t], B = LEFT ? xv[t] : wv[t];
+      cr = __builtin_amdgcn_mfma_f32_16x16x4f32(A.x, B.x, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f32_16x16x4f32(A.x, B.y, ci, 0, 0, 0);
+      cr = __builtin_amdgcn_mfma_f32_16x16x4f32(-A.y, B.y, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f32_16x16x4f32(A.y, B.x, ci, 0, 0, 0);
+    }
+  }
+  // lane (line, g) holds rows 4 g + e of column `line`
+  if (wave > 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) partial[wave - 1][64 * e + lane] = mkcf(cr[e], ci[e]);
+  }
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cf v = mkcf(cr[e], ci[e]);
+#pragma unroll
+      for (int h = 0; h < 3; ++h) v = cadd(v, partial[h][64 * e + lane]);
+      partial[0][64 * e + lane] = v;
+    }
+  }
+  __syncthreads();
+  // one output per thread (the envelope is some hundred float64 operations)
+  const int e = tid >> 6, row = i0 + 4 * g + e, col = j0 + line;
+  if (row < a.M && col < a.N) a.Y[(size_t)row * a.N + col] = dft_epilogue(a, partial[0][64 * e + lane], row, col, mean);
+}
+
+// more than DFT_MAX points: roots generated tile by tile
 template <bool LEFT>
-__global__ __launch_bounds__(256) void k_dft(const cf* __restrict__ X, cf* __restrict__ Y, int M, int N,
-                                             int inverse) {
+__global__ __launch_bounds__(256) void k_dft_any(DftArgs a) {
   __shared__ cf As[DFT_T][DFT_T + 1];
   __shared__ cf Bs[DFT_T][DFT_T + 1];
-  const int K = LEFT ? M : N;
+  const cf mean = a.sub_mean || a.add_mean ? mean_from_partials(a.part, (double)((long long)a.M * a.N)) : mkcf(0.f, 0.f);
+  const cf sub = a.sub_mean ? mean : mkcf(0.f, 0.f);
+  const int M = a.M, N = a.N, K = LEFT ? M : N;
   const int i0 = blockIdx.y * DFT_T, j0 = blockIdx.x * DFT_T;
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
   float ar[2][2] = {{0.f, 0.f}, {0.f, 0.f}}, ai[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
@@ -1928,11 +2075,11 @@ __global__ __launch_bounds__(256) void k_dft(const cf* __restrict__ X, cf* __res
       const int r = e / DFT_T, c = e % DFT_T;
       const int gi = i0 + r, gk = k0 + c;
       cf v = mkcf(0.f, 0.f);
-      if (gi < M && gk < K) v = LEFT ? dft_twiddle(gi, gk, K, inverse) : X[(size_t)gi * N + gk];
+      if (gi < M && gk < K) v = LEFT ? dft_twiddle(gi, gk, K, a.inverse) : csub(a.X[(size_t)gi * N + gk], sub);
       As[r][c] = v;
       const int hk = k0 + r, gj = j0 + c;
       cf u = mkcf(0.f, 0.f);
-      if (hk < K && gj < N) u = LEFT ? X[(size_t)hk * N + gj] : dft_twiddle(hk, gj, K, inverse);
+      if (hk < K && gj < N) u = LEFT ? csub(a.X[(size_t)hk * N + gj], sub) : dft_twiddle(hk, gj, K, a.inverse);
       Bs[r][c] = u;
     }
     __syncthreads();
@@ -1940,13 +2087,13 @@ __global__ __launch_bounds__(256) void k_dft(const cf* __restrict__ X, cf* __res
     for (int k = 0; k < DFT_T; ++k) {
       const cf a0 = As[2 * ty][k], a1 = As[2 * ty + 1][k];
       const cf b0 = Bs[k][2 * tx], b1 = Bs[k][2 * tx + 1];
-      const cf a[2] = {a0, a1}, b[2] = {b0, b1};
+      const cf av[2] = {a0, a1}, bv[2] = {b0, b1};
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          ar[u][v] += a[u].x * b[v].x - a[u].y * b[v].y;
-          ai[u][v] += a[u].x * b[v].y + a[u].y * b[v].x;
+          ar[u][v] += av[u].x * bv[v].x - av[u].y * bv[v].y;
+          ai[u][v] += av[u].x * bv[v].y + av[u].y * bv[v].x;
         }
     }
     __syncthreads();
@@ -1956,7 +2103,7 @@ __global__ __launch_bounds__(256) void k_dft(const cf* __restrict__ X, cf* __res
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
       const int gi = i0 + 2 * ty + u, gj = j0 + 2 * tx + v;
-      if (gi < M && gj < N) Y[(size_t)gi * N + gj] = mkcf(ar[u][v], ai[u][v]);
+      if (gi < M && gj < N) a.Y[(size_t)gi * N + gj] = dft_epilogue(a, mkcf(ar[u][v], ai[u][v]), gi, gj, mean);
     }
 }
 
@@ -2049,12 +2196,11 @@ __global__ __launch_bounds__(256) void k_lin_right(const cf* __restrict__ T, con
 }
 
 // float64 partial sums of the object (re, im) per block, fixed grid
-constexpr int MEAN_BLOCKS = 256;
-static_assert(MEAN_BLOCKS <= CONSTRAINT_PARTS, "mean partials share the constraint partial buffer");
 __global__ __launch_bounds__(256) void k_complex_sum_partial(const cf* __restrict__ obj, long long npix,
                                                              double* __restrict__ part) {
   __shared__ double sr[256], si[256];
   double a = 0.0, b = 0.0;
+#pragma unroll 4
   for (long long p = (long long)blockIdx.x * 256 + threadIdx.x; p < npix; p += (long long)MEAN_BLOCKS * 256) {
     a += (double)obj[p].x;
     b += (double)obj[p].y;
@@ -2075,68 +2221,30 @@ __global__ __launch_bounds__(256) void k_complex_sum_partial(const cf* __restric
   }
 }
 
-__device__ __forceinline__ cf mean_from_partials(const double* part, long long npix) {
-  double a = 0.0, b = 0.0;
-  for (int k = 0; k < MEAN_BLOCKS; ++k) {
-    a += part[2 * k];
-    b += part[2 * k + 1];
-  }
-  return mkcf((float)(a / (double)npix), (float)(b / (double)npix));
-}
-
-// sign = -1: O -= mean; sign = +1: O += mean
-__global__ __launch_bounds__(256) void k_shift_by_mean(cf* __restrict__ obj, long long npix,
-                                                       const double* __restrict__ part, float sign) {
-  __shared__ cf m_sh;
-  if (threadIdx.x == 0) m_sh = mean_from_partials(part, npix);
-  __syncthreads();
-  const cf m = m_sh;
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    const cf o = obj[p];
-    obj[p] = mkcf(o.x + sign * m.x, o.y + sign * m.y);
-  }
-}
-
-// spectrum times env(|q|) / (Px Py) (the inverse transform's normalisation),
-// env evaluated in float64 as the reference evaluates it
-__global__ __launch_bounds__(256) void k_butterworth_env(cf* __restrict__ spec, int Px, int Py, double dx,
-                                                         double dy, double q_lowpass, double q_highpass,
-                                                         double order) {
-  const long long npix = (long long)Px * Py;
-  const double vx = 1.0 / (Px * dx), vy = 1.0 / (Py * dy);
-  const double norm = 1.0 / ((double)Px * (double)Py);
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
-       p += (long long)gridDim.x * blockDim.x) {
-    const int x = (int)(p / Py), y = (int)(p % Py);
-    const int kx = x < (Px - 1) / 2 + 1 ? x : x - Px;  // numpy fftfreq order
-    const int ky = y < (Py - 1) / 2 + 1 ? y : y - Py;
-    const double qx = kx * vx, qy = ky * vy;
-    const double qr = sqrt(qx * qx + qy * qy);
-    double env = 1.0;
-    if (q_highpass != 0.0) env *= 1.0 - 1.0 / (1.0 + pow(qr / q_highpass, 2.0 * order));
-    if (q_lowpass != 0.0) env *= 1.0 / (1.0 + pow(qr / q_lowpass, 2.0 * order));
-    const double f = env * norm;
-    const cf v = spec[p];
-    spec[p] = mkcf((float)((double)v.x * f), (float)((double)v.y * f));
-  }
+template <bool LEFT> void launch_dft(const DftArgs& a, hipStream_t stream) {
+  const int n = LEFT ? a.M : a.N;
+  if (n <= DFT_MAX)
+    hipLaunchKernelGGL(k_dft<LEFT>, dim3((a.N + 15) / 16, (a.M + 15) / 16), dim3(256), (size_t)n * sizeof(cf), stream, a);
+  else
+    hipLaunchKernelGGL(k_dft_any<LEFT>, dim3((a.N + DFT_T - 1) / DFT_T, (a.M + DFT_T - 1) / DFT_T), dim3(256), 0, stream,
+                       a);
 }
 
 // tmp: Px * Py * 8 bytes; part: MEAN_BLOCKS * 16 bytes
 int launch_object_butterworth(cf* obj, int Px, int Py, double q_lowpass, double q_highpass, double order,
                               double dx, double dy, void* tmp, double* part, hipStream_t stream) {
-  const long long npix = (long long)Px * Py;
-  cf* t = (cf*)tmp;
-  const dim3 g2((Py + DFT_T - 1) / DFT_T, (Px + DFT_T - 1) / DFT_T), b2(256);
-  const dim3 g1(grid_for(npix, 256)), b1(256);
-  hipLaunchKernelGGL(k_complex_sum_partial, dim3(MEAN_BLOCKS), dim3(256), 0, stream, obj, npix, part);
-  hipLaunchKernelGGL(k_shift_by_mean, g1, b1, 0, stream, obj, npix, part, -1.f);
-  hipLaunchKernelGGL(k_dft<true>, g2, b2, 0, stream, obj, t, Px, Py, 0);
-  hipLaunchKernelGGL(k_dft<false>, g2, b2, 0, stream, t, obj, Px, Py, 0);
-  hipLaunchKernelGGL(k_butterworth_env, g1, b1, 0, stream, obj, Px, Py, dx, dy, q_lowpass, q_highpass, order);
-  hipLaunchKernelGGL(k_dft<true>, g2, b2, 0, stream, obj, t, Px, Py, 1);
-  hipLaunchKernelGGL(k_dft<false>, g2, b2, 0, stream, t, obj, Px, Py, 1);
-  hipLaunchKernelGGL(k_shift_by_mean, g1, b1, 0, stream, obj, npix, part, 1.f);
+  hipLaunchKernelGGL(k_complex_sum_partial, dim3(MEAN_BLOCKS), dim3(256), 0, stream, obj, (long long)Px * Py, part);
+  DftArgs a{};
+  a.M = Px; a.N = Py; a.part = part; a.dx = dx; a.dy = dy;
+  a.q_lowpass = q_lowpass; a.q_highpass = q_highpass; a.order = order;
+  a.X = obj; a.Y = (cf*)tmp; a.sub_mean = 1;
+  launch_dft<true>(a, stream);
+  a.X = (const cf*)tmp; a.Y = obj; a.sub_mean = 0; a.envelope = 1;
+  launch_dft<false>(a, stream);
+  a.X = obj; a.Y = (cf*)tmp; a.envelope = 0; a.inverse = 1;
+  launch_dft<true>(a, stream);
+  a.X = (const cf*)tmp; a.Y = obj; a.add_mean = 1;
+  launch_dft<false>(a, stream);
   return check_launch("k_dft");
 }
 
