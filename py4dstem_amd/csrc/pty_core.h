@@ -356,6 +356,15 @@ template <class T> PTY_HD T uniform_load(const T* p, unsigned i) {
 #endif
 }
 
+// a value that is the same for every lane of a wave
+PTY_HD int wave_uniform(int i) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_readfirstlane(i);
+#else
+  return i;
+#endif
+}
+
 // wrapi for a value known to lie in [-n, 2n): one conditional correction
 // per side instead of an integer division
 PTY_HD int wrap1(int a, int n) {
@@ -366,6 +375,76 @@ PTY_HD int wrap1(int a, int n) {
 // wrapi with the division only off the common path (an index already in
 // [0, n) is returned as is)
 PTY_HD int wrapi_fast(int a, int n) { return (unsigned)a < (unsigned)n ? a : wrapi(a, n); }
+
+// cos(2 pi m / 128), m = 0 .. 32; the other roots of unity follow by symmetry
+constexpr double COS128[33] = {
+    1.0, 0.9987954562051724, 0.9951847266721969, 0.989176509964781,
+    0.9807852804032304, 0.970031253194544, 0.9569403357322088, 0.9415440651830208,
+    0.9238795325112867, 0.9039892931234433, 0.881921264348355, 0.8577286100002721,
+    0.8314696123025452, 0.8032075314806449, 0.773010453362737, 0.7409511253549591,
+    0.7071067811865476, 0.6715589548470184, 0.6343932841636455, 0.5956993044924334,
+    0.5555702330196022, 0.5141027441932218, 0.47139673682599764, 0.4275550934302821,
+    0.3826834323650898, 0.33688985339222005, 0.2902846772544624, 0.2429801799032639,
+    0.19509032201612828, 0.14673047445536175, 0.0980171403295606, 0.049067674327418015,
+    0.0,
+};
+constexpr double cos128(int m) {
+  m = (m % 128 + 128) % 128;
+  if (m > 64) m = 128 - m;
+  return m <= 32 ? COS128[m] : -COS128[64 - m];
+}
+
+// Twiddles of the column passes of S = 64 and 128 px frames.  A column's
+// position in its line is the same for a whole wave there (lanes are
+// consecutive columns), so the N1 factors are scalar operands: read through
+// the scalar cache, they take neither LDS bandwidth nor vector registers nor
+// a wait behind the other waves' LDS traffic (2,048 positions of 64 px: 51.7
+// to 49.2 us a launch).
+template <int S> struct ColTwiddles {
+  static constexpr int N1 = Geo<S>::N1, N2 = Geo<S>::N2;
+  float a[N2][N1][2];   // forward A pass of line position n2: W^(n2 k1)
+  float b[N1][N2][2];   // inverse B' pass of k1: conj W^(n2 k1)
+  float bs[N1][N2][2];  // times 1 / S^2
+  constexpr ColTwiddles() : a(), b(), bs() {
+    for (int n2 = 0; n2 < N2; ++n2)
+      for (int k1 = 0; k1 < N1; ++k1) {
+        const int m = n2 * k1 * (128 / S);
+        const float c = (float)cos128(m), sn = (float)cos128(m - 32), k = 1.0f / (float)(S * S);
+        a[n2][k1][0] = c;
+        a[n2][k1][1] = -sn;
+        b[k1][n2][0] = c;
+        b[k1][n2][1] = sn;
+        bs[k1][n2][0] = c * k;
+        bs[k1][n2][1] = sn * k;
+      }
+  }
+};
+template <int S> constexpr ColTwiddles<S> COL_TWIDDLES = ColTwiddles<S>();
+
+// One 8-byte LDS access.  As relaxed atomics of a wave's scope these are the
+// plain ds_read_b64 and ds_write_b64, which the compiler would otherwise pair
+// into ds_read2_b64 and ds_write2_b64: a compute unit moves 216 bytes a clock
+// with the single loads and 127 with the paired ones (85 and 79 storing).  A
+// launch of 2,048 positions of 64 px went from 49.2 to 44.5 us with it, one of
+// 1,024 of 128 px from 113.9 to 108.9 us.  They keep their order among all
+// memory accesses: loads from elsewhere go in front of a run of them, not
+// between.
+PTY_HD cf lds_ld(const cf* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(cf, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_WAVEFRONT));
+#else
+  return *p;
+#endif
+}
+PTY_HD void lds_st(cf* p, cf v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+#else
+  *p = v;
+#endif
+}
 
 // Passes on one line (a row or a column) of a frame.  v[] is the thread's
 // register block; for A passes v[m] sits at line position n2 + N2*m, for B
@@ -379,20 +458,23 @@ template <int S> struct Pass {
   // at one base address) and at TW_B + k1 (N2 + 1) + n2 (the B' pass reads N2
   // values at one base), so every twiddle load is base + immediate offset.
   // The one-word pad per table row keeps the lanes of a row pass (which
-  // differ in n2, or k1) on distinct LDS banks.  A third copy at TW_BS holds
-  // the B' layout times 1/S^2, for the last inverse pass of a transform whose
-  // output carries the ifft2 normalisation (a power of two: scaling the
-  // twiddles is exact, and every later step is a sum or a product by a
-  // constant, so the result equals the scaled-after one bit for bit).
+  // differ in n2, or k1) on distinct LDS banks.  Where a column pass cannot
+  // take scalar twiddles (32 px: a wave holds two line positions), a third
+  // copy at TW_BS holds the B' layout times 1/S^2, for the last inverse pass
+  // of a transform whose output carries the ifft2 normalisation (a power of
+  // two: scaling the twiddles is exact, and every later step is a sum or a
+  // product by a constant, so the result equals the scaled-after one bit for
+  // bit).
+  static constexpr bool SCALAR_COLS = S % 64 == 0;
   static constexpr int TW_A = N2 * (N1 + 1);
   static constexpr int TW_BS = TW_A + N1 * (N2 + 1);
-  static constexpr int TW_WORDS = TW_BS + N1 * (N2 + 1);
+  static constexpr int TW_WORDS = SCALAR_COLS ? TW_BS : TW_BS + N1 * (N2 + 1);
   template <bool INV> static PTY_HD void A(int n2, cf* v, const cf* tw) {
     if (!INV) {
       dft<N1, false>(v);
       const cf* w = tw + n2 * (N1 + 1);
 #pragma unroll
-      for (int k1 = 1; k1 < N1; ++k1) v[k1] = cmul(v[k1], w[k1]);
+      for (int k1 = 1; k1 < N1; ++k1) v[k1] = cmul(v[k1], lds_ld(w + k1));
     } else {
       dft<N1, true>(v);
     }
@@ -408,19 +490,48 @@ template <int S> struct Pass {
         const cf* w = tw + (SCALED ? TW_BS : TW_A) + (R * t + g) * (N2 + 1);  // k1 = R t + g
         if (SCALED) u[0] = cscale(u[0], 1.0f / (float)(S * S));
 #pragma unroll
-        for (int n2 = 1; n2 < N2; ++n2) u[n2] = cmul(u[n2], cconj(w[n2]));
+        for (int n2 = 1; n2 < N2; ++n2) u[n2] = cmul(u[n2], cconj(lds_ld(w + n2)));
       }
     }
   }
   // twiddles for the inverse A' pass are applied in B'; the forward A pass
   // applies its own.  (Inverse: B' multiplies V[k1][n2] by conj W^(n2 k1).)
+
+  // the same passes along columns: q, the position in the line, is the same
+  // for the whole wave when SCALAR_COLS
+  static PTY_HD cf col_tw(const float* w, unsigned i) { return mkcf(uniform_load(w, 2 * i), uniform_load(w, 2 * i + 1)); }
+  template <bool INV> static PTY_HD void colA(int q, cf* v, const cf* tw) {
+    if constexpr (INV || !SCALAR_COLS) {
+      A<INV>(q, v, tw);
+    } else {
+      const float* w = &COL_TWIDDLES<S>.a[wave_uniform(q)][0][0];
+      dft<N1, false>(v);
+#pragma unroll
+      for (int k1 = 1; k1 < N1; ++k1) v[k1] = cmul(v[k1], col_tw(w, k1));
+    }
+  }
+  template <bool INV, bool SCALED = false> static PTY_HD void colB(int q, cf* v, const cf* tw) {
+    if constexpr (!INV || !SCALAR_COLS) {
+      B<INV, SCALED>(q, v, tw);
+    } else {
+      const float* w = SCALED ? &COL_TWIDDLES<S>.bs[R * wave_uniform(q)][0][0] : &COL_TWIDDLES<S>.b[R * wave_uniform(q)][0][0];
+#pragma unroll
+      for (int g = 0; g < R; ++g) {
+        cf* u = v + g * N2;
+        dft<N2, true>(u);
+        if (SCALED) u[0] = cscale(u[0], 1.0f / (float)(S * S));
+#pragma unroll
+        for (int n2 = 1; n2 < N2; ++n2) u[n2] = cmul(u[n2], col_tw(w, g * N2 + n2));
+      }
+    }
+  }
 };
 
 // LDS access policy used by the GPU kernels (the emulator supplies a checking one)
 struct LdsPtr {
   cf* p;
-  PTY_HD cf ld(int i) const { return p[i]; }
-  PTY_HD void st(int i, cf v) const { p[i] = v; }
+  PTY_HD cf ld(int i) const { return lds_ld(p + i); }
+  PTY_HD void st(int i, cf v) const { lds_st(p + i, v); }
 };
 
 // ---------------------------------------------------------------------------
@@ -598,7 +709,7 @@ template <int S> struct Fused {
     const int cc = F::col_line(tid), t = F::col_q(tid);
 #pragma unroll
     for (int j = 0; j < N1; ++j) r.v[j] = lds.ld(F::at(N1 * t + j, cc));
-    P::template B<INV, SCALED>(t, r.v, tw);
+    P::template colB<INV, SCALED>(t, r.v, tw);
 #pragma unroll
     for (int j = 0; j < N1; ++j) lds.st(F::at(N1 * t + j, cc), r.v[j]);
   }
@@ -610,7 +721,7 @@ template <int S> struct Fused {
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
 #pragma unroll
     for (int m = 0; m < N1; ++m) r.v[m] = lds.ld(F::at(n2 + N2 * m, cc));
-    P::template A<true>(n2, r.v, tw);
+    P::template colA<true>(n2, r.v, tw);
     if (SCALE) {
       const float s = 1.0f / (float)(S * S);
 #pragma unroll
@@ -674,7 +785,7 @@ template <int S> struct Fused {
 #pragma unroll
       for (int m = 0; m < N1; ++m) r.v[m] = cmul(r.v[m], expi(elem(a.object_pot, offset(m))));
     }
-    P::template A<false>(n2, r.v, tw);
+    P::template colA<false>(n2, r.v, tw);
 #pragma unroll
     for (int m = 0; m < N1; ++m) lds.st(F::at(n2 + N2 * m, cc), r.v[m]);
   }
@@ -744,7 +855,7 @@ template <int S> struct Fused {
       r.v[m] = cadd(cscale(psi, a.proj_c), cscale(e, a.proj_y));
       w_b[i * S + cc] = cadd(cscale(e, a.proj_x), cscale(psi, a.proj_a));
     }
-    P::template A<false>(n2, r.v, tw);
+    P::template colA<false>(n2, r.v, tw);
 #pragma unroll
     for (int m = 0; m < N1; ++m) lds.st(F::at(n2 + N2 * m, cc), r.v[m]);
   }
@@ -872,25 +983,40 @@ template <int S> struct Fused {
       const int i = n2 + N2 * m;
       r.v[m] = cconjmul(a.object[object_offset(a, r, i, cc)], chi_b[i * S + cc]);
     }
-    P::template A<false>(n2, r.v, tw);
+    P::template colA<false>(n2, r.v, tw);
 #pragma unroll
     for (int m = 0; m < N1; ++m) lds.st(F::at(n2 + N2 * m, cc), r.v[m]);
   }
 
-  // probe gradient, last phase: row pass B completes fft2(g); multiply by the
-  // conjugate ramp held in the LDS table; store in kernel layout
-  template <class L> static PTY_HD void p_pgrad_out(int tid, const FusedArgs& a, int b, Regs& r,
-                                                    L lds, const cf* tw) {
+  // probe gradient, last phases: row pass B completes fft2(g); multiply by the
+  // conjugate ramp held in the LDS table; through the rows of the frame that
+  // this wave owns into kernel layout, two elements a lane (a thread's own N1
+  // elements are 128 contiguous bytes at 128 px: 64 cache lines to a store)
+  template <class L> static PTY_HD void p_pgrad_rowB(int tid, Regs& r, L lds, const cf* tw) {
     const int rr = F::row_line(tid), t = F::row_q(tid);
 #pragma unroll
     for (int j = 0; j < N1; ++j) r.v[j] = lds.ld(F::at(rr, N1 * t + j));
     P::template B<false>(t, r.v, tw);
     const cf ex = lds.ld(RAMP + F::kidx(rr));
-    cf* out = a.pgrad_out + (size_t)b * S * S + rr * S + N1 * t;
 #pragma unroll
     for (int j = 0; j < N1; ++j) {
       const cf e = cmul(ex, lds.ld(RAMP + S + F::kidx(N1 * t + j)));
-      out[j] = cmul(r.v[j], e);
+      lds.st(F::at(rr, N1 * t + j), cmul(r.v[j], e));
+    }
+  }
+  template <class L> static PTY_HD void p_pgrad_out(int tid, const FusedArgs& a, int b, Regs& r, L lds) {
+    cf* out = a.pgrad_out + (size_t)b * S * S;
+#pragma unroll
+    for (int k = 0; k < N1 / 2; ++k) {
+      const unsigned e = tid / 64 * (64 * N1) + 2 * (k * 64 + tid % 64);
+      r.v[2 * k] = lds.ld(F::at(e / S, e % S));
+      r.v[2 * k + 1] = lds.ld(F::at(e / S, e % S) + 1);
+    }
+#pragma unroll
+    for (int k = 0; k < N1 / 2; ++k) {
+      const unsigned e = tid / 64 * (64 * N1) + 2 * (k * 64 + tid % 64);
+      elem(out, e) = r.v[2 * k];
+      elem(out, e + 1) = r.v[2 * k + 1];
     }
   }
 
@@ -1118,7 +1244,9 @@ template <int S, class Run> PTY_HD void probe_grad_position(Run& run, const Fuse
   run.barrier();
   run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::template p_rowA<false>(tid, r, lds, tw); });
   run.wave_barrier();
-  run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::p_pgrad_out(tid, a, b, r, lds, tw); });
+  run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::p_pgrad_rowB(tid, r, lds, tw); });
+  run.wave_barrier();
+  run.phase([&](int tid, Regs& r, auto lds, const cf*) { K::p_pgrad_out(tid, a, b, r, lds); });
   run.barrier();  // the ramp table and frame are rewritten by the next position
 }
 
@@ -1265,7 +1393,7 @@ template <int S> struct PosCorr {
       PTY_CHECK(row >= 0 && row < a.Px && col >= 0 && col < a.Py, "object index out of range");
       r.v[m] = cmul(ps_b[i * S + cc], a.object[(unsigned)row * (unsigned)a.Py + (unsigned)col]);
     }
-    P::template A<false>(n2, r.v, tw);
+    P::template colA<false>(n2, r.v, tw);
 #pragma unroll
     for (int m = 0; m < N1; ++m) lds.st(F::at(n2 + N2 * m, cc), r.v[m]);
   }

@@ -396,8 +396,14 @@ __device__ __forceinline__ void fft2_rowB_store(int tid, typename Fused<S>::Regs
 #pragma unroll
   for (int k = 0; k < F::N1 / 2; ++k) {
     const int e = 2 * (k * F::T + tid);
-    dst[e] = lds.ld(F::at(e / S, e % S));
-    dst[e + 1] = lds.ld(F::at(e / S, e % S) + 1);
+    r.v[2 * k] = lds.ld(F::at(e / S, e % S));
+    r.v[2 * k + 1] = lds.ld(F::at(e / S, e % S) + 1);
+  }
+#pragma unroll
+  for (int k = 0; k < F::N1 / 2; ++k) {
+    const int e = 2 * (k * F::T + tid);
+    dst[e] = r.v[2 * k];
+    dst[e + 1] = r.v[2 * k + 1];
   }
 }
 
@@ -449,8 +455,14 @@ __device__ __forceinline__ void fft2_body(const cf* __restrict__ in, cf* __restr
 #pragma unroll
       for (int k = 0; k < F::N1 / 2; ++k) {
         const int e = 2 * (k * F::T + tid);
-        lds.st(F::at(e / S, e % S), src[e]);
-        lds.st(F::at(e / S, e % S) + 1, src[e + 1]);
+        r.v[2 * k] = src[e];
+        r.v[2 * k + 1] = src[e + 1];
+      }
+#pragma unroll
+      for (int k = 0; k < F::N1 / 2; ++k) {
+        const int e = 2 * (k * F::T + tid);
+        lds.st(F::at(e / S, e % S), r.v[2 * k]);
+        lds.st(F::at(e / S, e % S) + 1, r.v[2 * k + 1]);
       }
       __syncthreads();
 #pragma unroll
