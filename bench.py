@@ -11,8 +11,8 @@ HBM.  Prints one JSON line.
 (square scans 32..96 positions per side, half 64 px and half 128 px frames,
 defocus 100..400 A, 30 iterations, mini-batch and stage size from the
 autotuner) advanced together by MultiPtychography (one launch per stage for
-all problems, one graph replay per iteration) against the same solves run one
-after another with reconstruct(); prints aggregate position-updates/s.
+all problems) against the same solves run one after another with
+reconstruct(); prints aggregate position-updates/s.
 
 ``--workload positions`` times the production workload with position
 correction on (reconstruct(fix_positions=False)); ``--workload projection``
@@ -225,7 +225,7 @@ def bench_many(args):
         "config": {
             "workload": f"{len(items)} independent GD ptychography reconstructions, square scans "
                         "32..96 per side, frames " + "/".join(map(str, frames)) +
-                        f" px, {num_iter} iterations, batched in one graph replay per iteration",
+                        f" px, {num_iter} iterations, batched in one launch per stage",
             "problems": len(items), "total_positions": npos,
             "mini_batch": {"min": min(batches), "max": max(batches)}, "stage": stage,
             "autotune_s_per_candidate": timings,

@@ -12,9 +12,9 @@
  *  - Complex arrays are complex64: interleaved float32 (re, im), 8-byte aligned.
  *  - All buffers are device memory owned by the caller; the library keeps no
  *    pointer after a call returns and allocates no device memory (the one
- *    static array of pty_gd_run_noalloc aside).  pty_multi_run creates
- *    runtime objects (a stream, two events, a graph) and waits for its work
- *    before returning; a pty_gd_run with pty_gd_params.pipeline set creates
+ *    static array of pty_gd_run_noalloc aside).  pty_multi_run waits for the
+ *    upload of its tables, and with use_graph for its work, before returning;
+ *    a pty_gd_run with pty_gd_params.pipeline set creates
  *    a second stream and four events once per device (kept until the
  *    process ends) and stays asynchronous; every other entry is
  *    asynchronous and creates none.
@@ -445,8 +445,8 @@ typedef struct pty_multi_problem {
 
 /* Advances `count` reconstructions (frames 64 and/or 128, any sizes) by
  * num_iter GD iterations.  Every stage of an iteration is one launch for all
- * problems; with use_graph the iteration's launch sequence is captured once
- * into a hipGraph and replayed num_iter times (returns after completion).
+ * problems.  With use_graph the call returns after completion, otherwise once
+ * the launches are queued.
  * Each problem's result is bitwise identical to its own pty_gd_run.  No
  * reference counterpart: the reference runs reconstructions one at a time. */
 size_t pty_multi_workspace_bytes(const pty_multi_problem* problems, int count);

@@ -3523,7 +3523,6 @@ int pty_multi_run(const pty_multi_problem* problems, int count, int num_iter, in
     d.run = (double*)(ws + L.run[i]); d.ppart = (double*)(ws + L.ppart[i]); d.cpart = (double*)(ws + L.cpart[i]);
   }
   ProblemDev* dP = (ProblemDev*)(ws + L.desc);
-  int* dIter = (int*)(ws + L.iter);
   int* dPl64 = (int*)(ws + L.plist64);
   int* dPl128 = (int*)(ws + L.plist128);
   hipError_t e = hipMemcpyAsync(dP, host.data(), sizeof(ProblemDev) * count, hipMemcpyHostToDevice, stream);
@@ -3537,51 +3536,17 @@ int pty_multi_run(const pty_multi_problem* problems, int count, int num_iter, in
                        stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);  // host tables are released on return
   if (e != hipSuccess) return fail(PTY_E_LAUNCH, "descriptor upload: %s", hipGetErrorString(e));
-  hipLaunchKernelGGL(km_iter_set, dim3(1), dim3(64), 0, stream, dIter, 0);
-  if ((rc = check_launch("km_iter_set"))) return rc;
-  if (!use_graph) {
-    for (int it = 0; it < num_iter; ++it)
-      if ((rc = multi_enqueue_iteration(plan, dP, dIter, dPl64, dPl128, stream))) return rc;
-    return PTY_OK;
-  }
-  // one iteration captured once, replayed num_iter times on a private stream
-  hipStream_t cs = nullptr;
-  hipEvent_t ready = nullptr, done = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventRecord(ready, stream);
-  if (e == hipSuccess) e = hipStreamWaitEvent(cs, ready, 0);
-  if (e == hipSuccess) e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    rc = multi_enqueue_iteration(plan, dP, dIter, dPl64, dPl128, cs);
-    hipError_t e2 = hipStreamEndCapture(cs, &graph);
-    if (!rc && e2 != hipSuccess) rc = fail(PTY_E_LAUNCH, "graph capture: %s", hipGetErrorString(e2));
-    if (!rc) {
-      e2 = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-      if (e2 != hipSuccess) rc = fail(PTY_E_LAUNCH, "graph instantiate: %s", hipGetErrorString(e2));
-    }
-    for (int it = 0; !rc && it < num_iter; ++it) {
-      e2 = hipGraphLaunch(exec, cs);
-      if (e2 != hipSuccess) rc = fail(PTY_E_LAUNCH, "graph launch: %s", hipGetErrorString(e2));
-    }
-    if (!rc) {
-      e2 = hipEventRecord(done, cs);
-      if (e2 == hipSuccess) e2 = hipStreamWaitEvent(stream, done, 0);
-      if (e2 != hipSuccess) rc = fail(PTY_E_LAUNCH, "graph join: %s", hipGetErrorString(e2));
-    }
-    (void)hipStreamSynchronize(cs);
-  } else {
-    rc = fail(PTY_E_LAUNCH, "graph setup: %s", hipGetErrorString(e));
-  }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (ready) (void)hipEventDestroy(ready);
-  if (done) (void)hipEventDestroy(done);
-  if (cs) (void)hipStreamDestroy(cs);
-  return rc;
+  // Launched one by one whatever use_graph says: an iteration captured into a
+  // graph and replayed was slower at every size (us, replayed / launched: two
+  // problems of 8 x 8 positions 721 / 503 at 4 iterations and 32,726 / 28,306
+  // at 256; twelve of 30 x 33, 64 and 128 px, 4,189 / 3,937 at 4 and 61,407 /
+  // 60,090 at 64), as a launch costs the host less than the shortest kernel
+  // takes, and a replay begins some 8 us after the one before it.
+  for (int it = 0; it < num_iter; ++it)
+    if ((rc = multi_enqueue_iteration(plan, dP, it, dPl64, dPl128, stream))) return rc;
+  if (use_graph && (e = hipStreamSynchronize(stream)) != hipSuccess)
+    return fail(PTY_E_LAUNCH, "batched run: %s", hipGetErrorString(e));
+  return PTY_OK;
 }
 
 }  // extern "C"

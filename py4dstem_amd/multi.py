@@ -3,7 +3,7 @@
 ``MultiPtychography`` takes preprocessed ``SingleslicePtychography`` objects
 (any mix of 64 and 128 pixel frames, any scan and object sizes) and runs
 their GD iterations with ``pty_multi_run``: one launch per stage for all
-problems and, by default, one captured hipGraph replayed per iteration.
+problems.
 Each problem's batch order is generated exactly as its own ``reconstruct()``
 would, and its result is bitwise identical to that sequential solve.
 
@@ -69,7 +69,9 @@ class MultiPtychography:
 
     def reconstruct(self, num_iter, reconstruct_kwargs=None, use_graph=True):
         """num_iter GD iterations of every problem.  reconstruct_kwargs: one
-        dict (shared) or a list of dicts with reconstruct() keywords."""
+        dict (shared) or a list of dicts with reconstruct() keywords.
+        use_graph: the native call returns after completion (the launches are
+        the same either way)."""
         if reconstruct_kwargs is None:
             reconstruct_kwargs = {}
         if isinstance(reconstruct_kwargs, dict):
