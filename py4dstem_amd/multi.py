@@ -23,6 +23,7 @@ import torch
 from . import _lib
 from . import autotune
 from ._lib import PtyMultiProblem, stream_handle
+from .ptychography import download
 
 
 class MultiPtychography:
@@ -78,8 +79,9 @@ class MultiPtychography:
             reconstruct_kwargs = [reconstruct_kwargs] * len(self.items)
         runs = self._runs(num_iter, reconstruct_kwargs)
         self.run_prepared(runs, num_iter, use_graph)
+        host = iter(download([t for p, run in zip(self.items, runs) for t in p._results(run)]))
         for p, run in zip(self.items, runs):
-            p._finish_run(run)
+            p._finish_run(run, (next(host), next(host), next(host)))
         return self
 
     @staticmethod
