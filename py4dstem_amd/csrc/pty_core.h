@@ -592,6 +592,7 @@ template <int S> struct Fused {
 
   struct Regs {
     cf v[N1];
+    cf w[N1];      // projection sets: partial new exit wave (column pass A layout)
     float amp[N1]; // this thread's measured amplitudes (row pass B layout),
                    // requested phases before the projection reads them
     double err;
@@ -834,26 +835,43 @@ template <int S> struct Fused {
   // overlap psi = P * O_patch, previous exit wave e (psi on the first
   // iteration), c psi + y e into the forward column pass, and the partial
   // new exit wave w = x e + a psi (the reference's left-to-right float32
-  // evaluation order) written over e: the same thread reads it back in the
-  // last phase (keeping it in registers through the transforms would spill)
+  // evaluation order), which stays in registers: at 128 px that spills 8 of
+  // them, and parking it in the exit wave's frame instead moved 256 KB more a
+  // position (2,968 positions: 581 against 428 us a launch)
   template <class L> static PTY_HD void p_proj_colA(int tid, const FusedArgs& a, int b, Regs& r,
                                                     L lds, const cf* tw) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-    p_colAinv_to_regs<L, false>(tid, r, lds, tw);
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
-    cf* ps_b = a.ps_out ? a.ps_out + (size_t)b * S * S : nullptr;
-    const cf* ex_b = a.chi_in + (size_t)b * S * S;
-    cf* w_b = a.chi_out + (size_t)b * S * S;
+    int col = r.y0 + F::fidx(cc);
+    col += col < 0 ? a.Py : 0;
+    col -= col >= a.Py ? a.Py : 0;
+    const CfBuf objb = cf_buf(a.object, (unsigned)a.Px * (unsigned)a.Py);
+    const CfBuf exb = cf_buf(a.chi_in + (size_t)b * S * S, S * S);
+    // the loads go out first: in flight during the inverse column pass
 #pragma unroll
     for (int m = 0; m < N1; ++m) {
-      const int i = n2 + N2 * m;
-      if (ps_b) ps_b[i * S + cc] = r.v[m];
-      const cf psi = cmul(r.v[m], a.object[object_offset(a, r, i, cc)]);
-      const cf e = a.exit_valid ? ex_b[i * S + cc] : psi;
+      const unsigned o = f32_bits(lds.ld(ROWS + n2 + N2 * m).x) + (unsigned)col;
+      PTY_CHECK(o < (unsigned)a.Px * (unsigned)a.Py && o == object_offset(a, r, n2 + N2 * m, cc),
+                "object index out of range");
+      r.w[m] = cf_ld(objb, o, 0u);
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+    p_colAinv_to_regs<L, false>(tid, r, lds, tw);
+    if (a.ps_out) {
+      const CfBuf psb = cf_buf(a.ps_out + (size_t)b * S * S, S * S);
+#pragma unroll
+      for (int m = 0; m < N1; ++m) cf_st(psb, n2 * S + cc, N2 * m * S, r.v[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < N1; ++m) {
+      const cf psi = cmul(r.v[m], r.w[m]);
+      const cf e = a.exit_valid ? cf_ld(exb, n2 * S + cc, N2 * m * S) : psi;
       r.v[m] = cadd(cscale(psi, a.proj_c), cscale(e, a.proj_y));
-      w_b[i * S + cc] = cadd(cscale(e, a.proj_x), cscale(psi, a.proj_a));
+      r.w[m] = cadd(cscale(e, a.proj_x), cscale(psi, a.proj_a));
     }
     P::template colA<false>(n2, r.v, tw);
 #pragma unroll
@@ -869,12 +887,9 @@ template <int S> struct Fused {
 #endif
     p_colAinv_to_regs(tid, r, lds, tw);
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
-    cf* ex_b = a.chi_out + (size_t)b * S * S;
+    const CfBuf exb = cf_buf(a.chi_out + (size_t)b * S * S, S * S);
 #pragma unroll
-    for (int m = 0; m < N1; ++m) {
-      const int o = (n2 + N2 * m) * S + cc;
-      ex_b[o] = cadd(ex_b[o], cscale(r.v[m], a.proj_b));
-    }
+    for (int m = 0; m < N1; ++m) cf_st(exb, n2 * S + cc, N2 * m * S, cadd(r.w[m], cscale(r.v[m], a.proj_b)));
   }
 
   // The probe spectrum in coalesced pieces: piece k (k < N1/2) of thread tid
