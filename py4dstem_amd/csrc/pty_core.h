@@ -295,17 +295,31 @@ PTY_HD CfBuf cf_buf(const cf* p, unsigned elems) {
   return b;
 }
 
-PTY_HD void cf_st(const CfBuf& b, unsigned vi, unsigned si, cf v) {
+// Where a frame's stores leave it (a launch's shifted probes and exit-wave
+// updates are written once and read by the next launch).  STREAM: past the
+// caches, so that a set larger than the 256 MB memory-side cache does not wash
+// through it.  THROUGH: through L2, so that no dirty lines are left to write
+// back when the launch ends, and kept in the memory-side cache.
+enum StorePolicy { STREAM = 2, THROUGH = 16 };  // nt; sc1
+
+template <StorePolicy P> PTY_HD void cf_st(const CfBuf& b, unsigned vi, unsigned si, cf v) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-  // cache policy 2: non-temporal (the frames are written once per
-  // position and read by another launch, so they should not evict the
-  // probe spectrum and the object from L2)
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), b.r, vi * 8u, si * 8u, 2);
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), b.r, vi * 8u, si * 8u, P);
 #else
   PTY_CHECK(vi + si < b.n, "buffer store out of range");
   b.p[vi + si] = v;
 #endif
+}
+// n stores, one every `step` elements
+template <int N> PTY_HD void cf_st_run(bool keep, const CfBuf& b, unsigned vi, unsigned step, const cf* v) {
+  if (keep) {
+#pragma unroll
+    for (int m = 0; m < N; ++m) cf_st<THROUGH>(b, vi, m * step, v[m]);
+  } else {
+#pragma unroll
+    for (int m = 0; m < N; ++m) cf_st<STREAM>(b, vi, m * step, v[m]);
+  }
 }
 
 PTY_HD cf cf_ld(const CfBuf& b, unsigned vi, unsigned si) {
@@ -576,6 +590,7 @@ struct FusedArgs {
   // 256 px frames: room for 16 partial errors per slot of the launch (from
   // slot b0), or null
   double* err_part;
+  int keep;  // the launch's frames stay in the memory-side cache (StorePolicy)
 };
 
 // exp(i v) as NumPy's complex64 exp(1j * v): (cos v, sin v)
@@ -761,9 +776,7 @@ template <int S> struct Fused {
     };
     auto store_ps = [&]() {
       if (a.ps_out) {
-        const CfBuf psb = cf_buf(a.ps_out + (size_t)b * S * S, S * S);
-#pragma unroll
-        for (int m = 0; m < N1; ++m) cf_st(psb, n2 * S + cc, N2 * m * S, r.v[m]);
+        cf_st_run<N1>(a.keep, cf_buf(a.ps_out + (size_t)b * S * S, S * S), n2 * S + cc, N2 * S, r.v);
       }
     };
     if constexpr (!POT) {
@@ -803,9 +816,7 @@ template <int S> struct Fused {
     for (int j = 0; j < N1; ++j) r.v[j] = lds.ld(F::at(rr, N1 * t + j));
     P::template B<false>(t, r.v, tw);
     if (a.fwd_out) {  // one uniform branch for the thread's whole row of F
-      const CfBuf farb = cf_buf(a.fwd_out + (size_t)b * S * S, S * S);
-#pragma unroll
-      for (int j = 0; j < N1; ++j) cf_st(farb, tid, j * T, r.v[j]);
+      cf_st_run<N1>(a.keep, cf_buf(a.fwd_out + (size_t)b * S * S, S * S), tid, T, r.v);
     }
     const float* fm = MASK ? a.fmask + rr * S + N1 * t : nullptr;
     double acc = 0.0;
@@ -862,9 +873,7 @@ template <int S> struct Fused {
 #endif
     p_colAinv_to_regs<L, false>(tid, r, lds, tw);
     if (a.ps_out) {
-      const CfBuf psb = cf_buf(a.ps_out + (size_t)b * S * S, S * S);
-#pragma unroll
-      for (int m = 0; m < N1; ++m) cf_st(psb, n2 * S + cc, N2 * m * S, r.v[m]);
+      cf_st_run<N1>(a.keep, cf_buf(a.ps_out + (size_t)b * S * S, S * S), n2 * S + cc, N2 * S, r.v);
     }
 #pragma unroll
     for (int m = 0; m < N1; ++m) {
@@ -887,9 +896,9 @@ template <int S> struct Fused {
 #endif
     p_colAinv_to_regs(tid, r, lds, tw);
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
-    const CfBuf exb = cf_buf(a.chi_out + (size_t)b * S * S, S * S);
 #pragma unroll
-    for (int m = 0; m < N1; ++m) cf_st(exb, n2 * S + cc, N2 * m * S, cadd(r.w[m], cscale(r.v[m], a.proj_b)));
+    for (int m = 0; m < N1; ++m) r.v[m] = cadd(r.w[m], cscale(r.v[m], a.proj_b));
+    cf_st_run<N1>(a.keep, cf_buf(a.chi_out + (size_t)b * S * S, S * S), n2 * S + cc, N2 * S, r.v);
   }
 
   // The probe spectrum in coalesced pieces: piece k (k < N1/2) of thread tid
@@ -1053,9 +1062,7 @@ template <int S> struct Fused {
   static PTY_HD void p_outputs(int tid, const FusedArgs& a, int b, Regs& r, L lds, const cf* tw) {
     p_colAinv_to_regs<L, !PRESCALED>(tid, r, lds, tw);
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
-    const CfBuf chib = cf_buf(a.chi_out + (size_t)b * S * S, S * S);
-#pragma unroll
-    for (int m = 0; m < N1; ++m) cf_st(chib, n2 * S + cc, N2 * m * S, r.v[m]);
+    cf_st_run<N1>(a.keep, cf_buf(a.chi_out + (size_t)b * S * S, S * S), n2 * S + cc, N2 * S, r.v);
   }
 };
 

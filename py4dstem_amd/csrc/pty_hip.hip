@@ -1623,10 +1623,21 @@ bool frame_supported(int S) { return S == 32 || S == 64 || S == 128; }
 // frames of the gradient-descent path: also 256 (line passes, pty_256.inc)
 bool frame_supported_gd(int S) { return frame_supported(S) || S == 256; }
 
-int launch_fused(const FusedArgs& a, int S, hipStream_t stream) {
+// Whether a launch's frames are written so that they stay in the 256 MB
+// memory-side cache for the launch that reads them.  Fused pass + scatter, us,
+// streamed / kept: 288 positions of 64 px 31.9 / 30.3 (19 MB), 1,024 48.8 /
+// 45.4 (67 MB), 2,048 93.3 / 85.0 (134 MB); 384 of 128 px 89.9 / 83.8 (101 MB),
+// 768 153.3 / 149.6 (201 MB), 1,024 202.3 / 212.2 (268 MB), 1,536 282 / 313
+// (403 MB).  Keeping a part of a larger set gained nothing.
+constexpr size_t KEEP_BYTES = (size_t)224 << 20;
+int frames_kept(size_t frames, int S) { return frames * S * S * sizeof(cf) <= KEEP_BYTES; }
+
+int launch_fused(const FusedArgs& a_, int S, hipStream_t stream) {
+  FusedArgs a = a_;
   const int grid = a.B - a.b0;
   if (grid <= 0) return PTY_OK;
   if (S == 256) return launch_fused256(a, stream);
+  a.keep = frames_kept((size_t)grid * (a.fwd_out ? 3 : 2), S);
   if (a.object_pot) {  // potential object (no detector mask: the caller rejects the pair)
     if (a.fmask) return fail(PTY_E_UNSUPPORTED, "detector masks with potential objects are not supported");
     if (S == 32) hipLaunchKernelGGL((k_fused<32, false, true>), dim3(grid), dim3(Frame<32>::T), 0, stream, a);
@@ -1644,18 +1655,22 @@ int launch_fused(const FusedArgs& a, int S, hipStream_t stream) {
   return check_launch("k_fused");
 }
 
-int launch_mixed(const FusedArgs& a, int S, hipStream_t stream) {
+int launch_mixed(const FusedArgs& a_, int S, hipStream_t stream) {
+  FusedArgs a = a_;
   const int grid = a.B - a.b0;
   if (grid <= 0) return PTY_OK;
+  a.keep = frames_kept((size_t)grid * a.K * 2, S);
   if (S == 32) hipLaunchKernelGGL(k_mixed<32>, dim3(grid), dim3(Frame<32>::T), 0, stream, a);
   else if (S == 64) hipLaunchKernelGGL(k_mixed<64>, dim3(grid), dim3(Frame<64>::T), 0, stream, a);
   else hipLaunchKernelGGL(k_mixed<128>, dim3(grid), dim3(Frame<128>::T), 0, stream, a);
   return check_launch("k_mixed");
 }
 
-int launch_projection(const FusedArgs& a, int S, hipStream_t stream) {
+int launch_projection(const FusedArgs& a_, int S, hipStream_t stream) {
+  FusedArgs a = a_;
   const int grid = a.B - a.b0;
   if (grid <= 0) return PTY_OK;
+  a.keep = frames_kept((size_t)grid * 2, S);
   if (S == 32) hipLaunchKernelGGL(k_projection<32>, dim3(grid), dim3(Frame<32>::T), 0, stream, a);
   else if (S == 64) hipLaunchKernelGGL(k_projection<64>, dim3(grid), dim3(Frame<64>::T), 0, stream, a);
   else hipLaunchKernelGGL(k_projection<128>, dim3(grid), dim3(Frame<128>::T), 0, stream, a);
@@ -3503,6 +3518,10 @@ int pty_multi_run(const pty_multi_problem* problems, int count, int num_iter, in
     rounds.insert(rounds.end(), plan.bsize[i].begin(), plan.bsize[i].end());
   }
   int* dRounds = (int*)(ws + L.rounds);
+  size_t words = 0;  // of all problems' frames: one launch writes them
+  for (int i = 0; i < count; ++i)
+    words += (size_t)2 * std::min(plan.stage[i], problems[i].params.max_batch) * problems[i].problem.S * problems[i].problem.S;
+  const int keep = words * sizeof(cf) <= KEEP_BYTES;
   for (int i = 0; i < count; ++i) {
     const pty_problem& p = problems[i].problem;
     const pty_gd_params& q = problems[i].params;
@@ -3510,6 +3529,7 @@ int pty_multi_run(const pty_multi_problem* problems, int count, int num_iter, in
     d.S = p.S; d.Px = p.Px; d.Py = p.Py; d.N = p.N; d.nbatch = (int)plan.bsize[i].size(); d.stage = plan.stage[i];
     d.fix_probe = q.fix_probe; d.fix_probe_com = q.fix_probe_com; d.pure_phase = q.pure_phase_object;
     d.use_mask = p.fov_mask_inverse != nullptr;
+    d.keep = keep;
     d.step = q.step_size; d.c1 = (float)(1.0 - (double)q.normalization_min); d.c2 = q.normalization_min;
     d.shrink = q.shrinkage_rad;
     d.norm = (double)(float)(p.mean_intensity * (float)p.N);
