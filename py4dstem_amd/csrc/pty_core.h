@@ -1362,9 +1362,12 @@ template <int S> struct PosCorr {
   static constexpr int N1 = F::N1, N2 = F::N2, T = F::T;
   static constexpr int LDS_TOTAL = F::LDS_WORDS;
 
-  // Register budget (1024 threads: 128 VGPRs): F is loaded at set-up and
-  // stays live; the amplitudes are loaded only for the second transform's
-  // last row passes and the sums exist only in the final phase.
+  // Register budget (1024 threads: 128 VGPRs): F is loaded behind the first
+  // transform's columns and stays live from there; the amplitudes are loaded
+  // only for the second transform's last row passes and the sums exist only
+  // in the final phase.  With F loaded at set-up the first transform's loads
+  // of P_shift and object went out a few at a time: 768 positions of 128 px
+  // 105 us a launch, 94 us now.
   struct Regs {
     cf v[N1];
     cf f[N1];      // F at this thread's row-pass-B positions
@@ -1374,7 +1377,7 @@ template <int S> struct PosCorr {
     int x0, y0, idx;
   };
 
-  // anchor of slot b; the loads of F stay in flight across the first transform
+  // anchor of slot b
   static PTY_HD void p_setup(int tid, const PosArgs& a, int b, Regs& r) {
     int idx = a.order ? a.order[b] : b;
     PTY_CHECK(idx >= 0 && idx < a.N, "order index out of range");
@@ -1382,10 +1385,16 @@ template <int S> struct PosCorr {
     r.idx = idx;
     r.x0 = wrapi((int)rintf(a.positions[2 * idx]), a.Px);
     r.y0 = wrapi((int)rintf(a.positions[2 * idx + 1]), a.Py);
+  }
+
+  // row pass A of the first transform; the loads of F, issued first, complete
+  // behind it
+  template <class L> static PTY_HD void p_rowA_far(int tid, const PosArgs& a, int b, Regs& r, L lds, const cf* tw) {
     const size_t modes = a.far_modes > 0 ? (size_t)a.far_modes : 1;  // 0: single mode
     const cf* Fb = a.far + (size_t)b * modes * S * S + tid;
 #pragma unroll
     for (int j = 0; j < N1; ++j) r.f[j] = Fb[(size_t)j * T];
+    Fused<S>::template p_rowA<false>(tid, r, lds, tw);
   }
 
   // row pass A of the second transform; the amplitude loads issued first
@@ -1402,7 +1411,8 @@ template <int S> struct PosCorr {
   template <int DX, int DY, class L>
   static PTY_HD void p_colA(int tid, const PosArgs& a, int b, Regs& r, L lds, const cf* tw) {
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
-    const cf* ps_b = a.ps + (size_t)b * S * S;
+    const CfBuf psb = cf_buf(a.ps + (size_t)b * S * S, S * S);
+    const CfBuf objb = cf_buf(a.object, (unsigned)a.Px * (unsigned)a.Py);
     int col = r.y0 + F::fidx(cc) + DY;
     col += col < 0 ? a.Py : 0;
     col -= col >= a.Py ? a.Py : 0;
@@ -1413,7 +1423,7 @@ template <int S> struct PosCorr {
       row += row < 0 ? a.Px : 0;
       row -= row >= a.Px ? a.Px : 0;
       PTY_CHECK(row >= 0 && row < a.Px && col >= 0 && col < a.Py, "object index out of range");
-      r.v[m] = cmul(ps_b[i * S + cc], a.object[(unsigned)row * (unsigned)a.Py + (unsigned)col]);
+      r.v[m] = cmul(cf_ld(psb, n2 * S + cc, N2 * m * S), cf_ld(objb, (unsigned)row * (unsigned)a.Py + (unsigned)col, 0u));
     }
     P::template colA<false>(n2, r.v, tw);
 #pragma unroll
@@ -1508,7 +1518,7 @@ PTY_HD void position_correction_position(Run& run, const PosArgs& a, int b) {
   run.barrier();
   run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { FK::template p_colB<false>(tid, r, lds, tw); });
   run.barrier();
-  run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { FK::template p_rowA<false>(tid, r, lds, tw); });
+  run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::p_rowA_far(tid, a, b, r, lds, tw); });
   run.wave_barrier();
   run.phase([&](int tid, Regs& r, auto lds, const cf* tw) { K::p_partial_x(tid, r, lds, tw); });
   run.barrier();
