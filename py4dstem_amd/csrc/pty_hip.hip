@@ -712,21 +712,25 @@ __device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, in
   for (int t = threadIdx.x; t < nb; t += blockDim.x) {
     int idx = a.order[b0 + t];
     idx = ((unsigned)idx < (unsigned)a.N) ? idx : 0;
-    sh.anchor[t] = make_int2(wrap1(wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px) - S / 2, a.Px),
-                             wrap1(wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py) - S / 2, a.Py));
+    sh.anchor[t] = make_int2(wrapi_fast(wrapi_fast((int)rintf(a.positions[2 * idx]), a.Px) - S / 2, a.Px),
+                             wrapi_fast(wrapi_fast((int)rintf(a.positions[2 * idx + 1]), a.Py) - S / 2, a.Py));
   }
   __syncthreads();
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int pix = blk * (R * 64) + lane;  // and 64 r beyond; S * S is a multiple of 256
   const unsigned Px = a.Px, Py = a.Py;
   const cf* chi = a.chi + (size_t)b0 * S * S + pix;
-  // window coordinates of probe pixel (i, j): corner-centred index ^ S/2
+  // window coordinates of probe pixel (i, j), corner-centred index ^ S/2, below
+  // Px and Py also where the frame is larger than the object (it then meets an
+  // object pixel several times)
   unsigned wi[R], wj[R];
   double re[R], im[R], so[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     wi[r] = (unsigned)((pix + 64 * r) >> __builtin_ctz(S)) ^ (unsigned)(S / 2);  // S a power of two
     wj[r] = (unsigned)((pix + 64 * r) & (S - 1)) ^ (unsigned)(S / 2);
+    if (Px < (unsigned)S) wi[r] %= Px;
+    if (Py < (unsigned)S) wj[r] %= Py;
     re[r] = im[r] = so[r] = 0.0;
   }
   const auto object = [&](int k, int r) {
