@@ -2703,9 +2703,11 @@ int gd_run(const pty_problem* problem, const pty_gd_params* params, const pty_po
         a.order = ob + s0; a.N = p.N; a.B = ns; a.Px = p.Px; a.Py = p.Py; a.b0 = 0;
         a.ps_out = ps_k; a.chi_out = chi_k; a.err = err + start + s0; a.fwd_out = far;
         a.fmask = p.fourier_mask;
-        // the scatter's object sums are not live during the fused pass of an
-        // unpipelined run: room for the partial errors of 256 px frames
-        a.err_part = !pipe && (long long)ns * 16 <= (long long)p.Px * p.Py ? (double*)grad : nullptr;
+        // the scatter's object sums are not live during the fused pass (the
+        // scatter beside it in a pipelined run is never a batch's last, so it
+        // writes the running sums instead): room for the partial errors of
+        // 256 px frames
+        a.err_part = (long long)ns * 16 <= (long long)p.Px * p.Py ? (double*)grad : nullptr;
         if ((rc = launch_fused(a, p.S, stream))) return rc;
         if (pipe && ((rc = hip_check(hipEventRecord(pipe->fused_done[k & 1], stream), "hipEventRecord")) ||
                      (rc = hip_check(hipStreamWaitEvent(gs, pipe->fused_done[k & 1], 0), "hipStreamWaitEvent"))))
