@@ -1412,7 +1412,6 @@ template <int S> struct PosCorr {
   static PTY_HD void p_colA(int tid, const PosArgs& a, int b, Regs& r, L lds, const cf* tw) {
     const int cc = F::col_line(tid), n2 = F::col_q(tid);
     const CfBuf psb = cf_buf(a.ps + (size_t)b * S * S, S * S);
-    const CfBuf objb = cf_buf(a.object, (unsigned)a.Px * (unsigned)a.Py);
     int col = r.y0 + F::fidx(cc) + DY;
     col += col < 0 ? a.Py : 0;
     col -= col >= a.Py ? a.Py : 0;
@@ -1423,7 +1422,8 @@ template <int S> struct PosCorr {
       row += row < 0 ? a.Px : 0;
       row -= row >= a.Px ? a.Px : 0;
       PTY_CHECK(row >= 0 && row < a.Px && col >= 0 && col < a.Py, "object index out of range");
-      r.v[m] = cmul(cf_ld(psb, n2 * S + cc, N2 * m * S), cf_ld(objb, (unsigned)row * (unsigned)a.Py + (unsigned)col, 0u));
+      // a plain load: the batch entry takes objects beyond a buffer's range
+      r.v[m] = cmul(cf_ld(psb, n2 * S + cc, N2 * m * S), a.object[(unsigned)row * (unsigned)a.Py + (unsigned)col]);
     }
     P::template colA<false>(n2, r.v, tw);
 #pragma unroll
