@@ -44,8 +44,10 @@ enum {
   PTY_OK = 0,
   PTY_E_ARG = -1,      /* bad size, null pointer or misalignment */
   PTY_E_UNSUPPORTED = -2, /* frame size not compiled, option not on this path, an
-                             object of 2^28 elements or more, or a staged batch
-                             beyond 2^31 elements */
+                             object of 2^28 elements or more (2^29 for the loss and
+                             the simulation; pty_position_correction_batch takes any
+                             of 32-bit element indices), or a staged batch beyond
+                             2^31 elements */
   PTY_E_LAUNCH = -3,   /* HIP launch / runtime error */
   PTY_E_WORKSPACE = -4 /* workspace too small */
 };

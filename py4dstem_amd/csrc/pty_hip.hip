@@ -71,6 +71,12 @@ int check_index_range(long long Px, long long Py, long long frames, long long S)
   return PTY_OK;
 }
 
+// entries that bound the object by its 32-bit byte range alone
+int check_object_bytes(long long Px, long long Py) {
+  if (Px * Py >= (1ll << 29)) return fail(PTY_E_UNSUPPORTED, "object %lldx%lld beyond 2^29 elements", Px, Py);
+  return PTY_OK;
+}
+
 bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
 inline hipStream_t st(pty_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
@@ -3252,6 +3258,7 @@ int pty_loss_gradients(const void* object, const void* probe, int Px, int Py, co
     return fail(PTY_E_ARG, "bad loss_gradients sizes");
   if (!object || !probe || !positions || !amplitudes || !order || !loss || !workspace)
     return fail(PTY_E_ARG, "null buffer in loss_gradients");
+  if (int rc = check_object_bytes(Px, Py)) return rc;
   const int M = num_slots;
   const int Bc = chunk < M ? chunk : M;
   const LossLayout L = loss_layout(S, Px, Py, M, Bc);
@@ -3334,6 +3341,7 @@ int pty_simulate_intensities(const void* probe_hat, const void* object, int Px, 
   if (!frame_supported(S)) return fail(PTY_E_UNSUPPORTED, "frame size S=%d not supported", S);
   if (Px < S || Py < S || N < 0) return fail(PTY_E_ARG, "bad simulate sizes");
   if (!probe_hat || !object || !positions || !out) return fail(PTY_E_ARG, "null buffer in simulate");
+  if (int rc = check_object_bytes(Px, Py)) return rc;
   if (N == 0) return PTY_OK;
   FusedArgs a{};
   a.probe_hat = (const cf*)probe_hat; a.object = (const cf*)object; a.positions = positions;
