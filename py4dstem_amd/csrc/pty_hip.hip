@@ -1710,7 +1710,7 @@ int launch_scatter(const GatherArgs& a, hipStream_t stream) {
                        plan.tiles_x * plan.tiles_y);
     return check_launch("k_gather");
   }
-  const dim3 grid(scatter_blocks(a.Px, a.Py)), blk(256);
+  const dim3 grid(scatter_blocks(plan)), blk(256);
   if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter<1>, grid, blk, 0, stream, a, plan);
   else hipLaunchKernelGGL(k_scatter<4>, grid, blk, 0, stream, a, plan);
   return check_launch("k_scatter");
@@ -1804,7 +1804,7 @@ int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStr
     return PTY_OK;
   }
   const ScatterPlan plan = scatter_plan(g.Px, g.Py);
-  const int ns = scatter_blocks(g.Px, g.Py);
+  const int ns = scatter_blocks(plan);
   const int rp = probe_pixels_per_lane(pa.S, nchunk), pix_blocks = pa.S * pa.S / (rp * PROBE_PIX);
   const dim3 grid(ns + pix_blocks * nchunk, K), blk(256);
   if (plan.rows_per_lane == 1 && rp == 1)
@@ -3543,7 +3543,7 @@ int pty_multi_run(const pty_multi_problem* problems, int count, int num_iter, in
     d.S = p.S; d.Px = p.Px; d.Py = p.Py; d.N = p.N; d.nbatch = (int)plan.bsize[i].size(); d.stage = plan.stage[i];
     d.fix_probe = q.fix_probe; d.fix_probe_com = q.fix_probe_com; d.pure_phase = q.pure_phase_object;
     d.use_mask = p.fov_mask_inverse != nullptr;
-    d.keep = keep;
+    d.keep = keep; d.scatter_rows = plan.scatter_rows[i];
     d.step = q.step_size; d.c1 = (float)(1.0 - (double)q.normalization_min); d.c2 = q.normalization_min;
     d.shrink = q.shrinkage_rad;
     d.norm = (double)(float)(p.mean_intensity * (float)p.N);
