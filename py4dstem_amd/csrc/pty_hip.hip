@@ -542,6 +542,21 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather(GatherArgs a, int nti
   gather_body(a, (int)blockIdx.x, (int)gridDim.x, ntiles, sh);
 }
 
+// what lies between one probe mode's arrays and the next one's
+struct ModeStride {
+  size_t frames, pixels, tiles;  // elements of the staged frames, object pixels, tile maxima
+  size_t part, probe;            // bytes of the probe partials, elements of the probe
+};
+
+__host__ __device__ inline GatherArgs gather_mode(GatherArgs g, const ModeStride& m, size_t k) {
+  g.ps += k * m.frames;
+  g.chi += k * m.frames;
+  g.grad += k * m.pixels;
+  g.spsum += k * m.pixels;
+  g.tilemax += k * m.tiles;
+  return g;
+}
+
 #include "pty_scatter.inc"
 
 // Correctly rounded float32 square root of x >= 0 (IEEE / NumPy semantics).
@@ -798,12 +813,6 @@ __device__ __forceinline__ void probe_partial_body(const ProbePartialArgs& a, in
   }
 }
 
-// what lies between one probe mode's arrays and the next one's
-struct ModeStride {
-  size_t frames, pixels, tiles;  // elements of the staged frames, object pixels, tile maxima
-  size_t part, probe;            // bytes of the probe partials, elements of the probe
-};
-
 __global__ __launch_bounds__(256) void k_probe_partial(ProbePartialArgs a) {
   __shared__ ProbeShared<4> sh;
   probe_partial_body<4>(a, blockIdx.x, blockIdx.y, sh);
@@ -822,11 +831,7 @@ __global__ __launch_bounds__(256) void k_scatter_probe(GatherArgs g, ScatterPlan
   const int b = (int)blockIdx.x;
   if (gridDim.y > 1) {
     const size_t k = blockIdx.y;
-    g.ps += k * m.frames;
-    g.chi += k * m.frames;
-    g.grad += k * m.pixels;
-    g.spsum += k * m.pixels;
-    g.tilemax += k * m.tiles;
+    g = gather_mode(g, m, k);
     pa.chi += k * m.frames;
     pa.part = (double*)((char*)pa.part + k * m.part);
   }
@@ -1703,16 +1708,26 @@ int launch_fft(const cf* in, cf* out, int batch, int S, bool inv, int natural, h
   return check_launch("k_fft2");
 }
 
-int launch_scatter(const GatherArgs& a, hipStream_t stream) {
-  const ScatterPlan plan = scatter_plan(a.Px, a.Py);
+// K probe modes share the launch (scatter_wide)
+ScatterPlan modes_plan(const GatherArgs& a, int K) {
+  const long long pixels = (long long)a.Px * a.Py * K;
+  return scatter_plan(a.Px, a.Py, scatter_wide(pixels, (long long)a.S * a.S * a.B * K) ? 4 : scatter_rows(a.Px, a.Py));
+}
+
+// the scatter of a stage, of K probe modes
+int launch_scatter(const GatherArgs& a, hipStream_t stream, int K = 1, const ModeStride& m = ModeStride{}) {
   if (!scatter_in_range(a.B, a.S)) {
-    hipLaunchKernelGGL(k_gather, dim3(gather_num_tiles(a.Px, a.Py)), dim3(GATHER_THREADS), 0, stream, a,
-                       plan.tiles_x * plan.tiles_y);
-    return check_launch("k_gather");
+    for (int k = 0; k < K; ++k) {
+      hipLaunchKernelGGL(k_gather, dim3(gather_num_tiles(a.Px, a.Py)), dim3(GATHER_THREADS), 0, stream,
+                         gather_mode(a, m, k), scatter_num_tiles(a.Px, a.Py));
+      if (int rc = check_launch("k_gather")) return rc;
+    }
+    return PTY_OK;
   }
-  const dim3 grid(scatter_blocks(plan)), blk(256);
-  if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter<1>, grid, blk, 0, stream, a, plan);
-  else hipLaunchKernelGGL(k_scatter<4>, grid, blk, 0, stream, a, plan);
+  const ScatterPlan plan = modes_plan(a, K);
+  const dim3 grid(scatter_blocks(plan), K), blk(256);
+  if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter<1>, grid, blk, 0, stream, a, plan, m);
+  else hipLaunchKernelGGL(k_scatter<4>, grid, blk, 0, stream, a, plan, m);
   return check_launch("k_scatter");
 }
 
@@ -1791,19 +1806,16 @@ int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStr
   const int nchunk = probe_nchunk(pa.B);
   if (!scatter_in_range(g.B, g.S)) {
     for (int k = 0; k < K; ++k) {
-      GatherArgs gk = g;
-      gk.ps += k * m.frames; gk.chi += k * m.frames; gk.grad += k * m.pixels; gk.spsum += k * m.pixels;
-      gk.tilemax += k * m.tiles;
       ProbePartialArgs pk = pa;
       pk.chi += k * m.frames; pk.part = (double*)((char*)pa.part + k * m.part);
-      int rc = launch_scatter(gk, stream);
+      int rc = launch_scatter(gather_mode(g, m, k), stream);
       if (rc) return rc;
       hipLaunchKernelGGL(k_probe_partial, dim3(pa.S * pa.S / (4 * PROBE_PIX), nchunk), dim3(256), 0, stream, pk);
       if ((rc = check_launch("k_probe_partial"))) return rc;
     }
     return PTY_OK;
   }
-  const ScatterPlan plan = scatter_plan(g.Px, g.Py);
+  const ScatterPlan plan = modes_plan(g, K);
   const int ns = scatter_blocks(plan);
   const int rp = probe_pixels_per_lane(pa.S, nchunk), pix_blocks = pa.S * pa.S / (rp * PROBE_PIX);
   const dim3 grid(ns + pix_blocks * nchunk, K), blk(256);
@@ -3018,12 +3030,7 @@ int mixed_run(const pty_problem* problem, const pty_gd_params* params, int K, co
       g.Px = p.Px; g.Py = p.Py; g.tiles_y = gather_tiles_y(p.Py); g.grad = grad; g.spsum = spsum; g.tilemax = tilemax;
       ProbeStep step{};
       if (q.fix_probe) {
-        for (int k = 0; k < K; ++k) {
-          GatherArgs gk = g;
-          gk.ps += k * ms.frames; gk.chi += k * ms.frames; gk.grad += k * ms.pixels; gk.spsum += k * ms.pixels;
-          gk.tilemax += k * ms.tiles;
-          if ((rc = launch_scatter(gk, stream))) return rc;
-        }
+        if ((rc = launch_scatter(g, stream, K, ms))) return rc;
       } else {  // every mode's scatter and probe partial sums in one launch
         const ProbePartialArgs pa{chi, obj, p.positions, ob, p.N, nb, p.S, p.Px, p.Py, (double*)(ws + L.ppart)};
         if ((rc = launch_scatter_probe(g, pa, stream, K, ms))) return rc;
