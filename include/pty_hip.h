@@ -93,8 +93,8 @@ int pty_forward_adjoint_batch(const void* probe_hat, const void* object, int Px,
  * (phase_base_class.py:1905-1968, _sum_overlapping_patches_bincounts, as
  * called at ptychographic_methods.py:1859-1886):
  *   grad = scatter(conj(ps) * chi), spsum = scatter(|ps|^2);
- *   tilemax[t] = max spsum over object tile t, pty_scatter_num_tiles(Px, Py)
- *   entries.  S may also be 32 (stitching of learned-initialiser patches). */
+ *   tilemax = max spsum over each of the launch's object tiles,
+ *   pty_scatter_num_tiles(Px, Py) entries (0 in those it has no tile for).  S may also be 32 (stitching of learned-initialiser patches). */
 int pty_scatter_num_tiles(int Px, int Py);
 int pty_scatter_patches(const void* ps, const void* chi, const float* positions, int N,
                         const int* order, int B, int S, int Px, int Py, void* grad, float* spsum,

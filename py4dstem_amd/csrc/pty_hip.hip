@@ -1708,10 +1708,12 @@ int launch_fft(const cf* in, cf* out, int batch, int S, bool inv, int natural, h
   return check_launch("k_fft2");
 }
 
-// K probe modes share the launch (scatter_wide)
-ScatterPlan modes_plan(const GatherArgs& a, int K) {
-  const long long pixels = (long long)a.Px * a.Py * K;
-  return scatter_plan(a.Px, a.Py, scatter_wide(pixels, (long long)a.S * a.S * a.B * K) ? 4 : scatter_rows(a.Px, a.Py));
+// of a stage of K probe modes
+ScatterPlan stage_plan(const GatherArgs& a, int K) {
+  const bool wide = scatter_wide((long long)a.Px * a.Py * K, (long long)a.S * a.S * a.B * K);
+  ScatterPlan plan = scatter_plan(a.Px, a.Py, wide ? 4 : scatter_rows(a.Px, a.Py));
+  plan.num_tiles = scatter_num_tiles(a.Px, a.Py);
+  return plan;
 }
 
 // the scatter of a stage, of K probe modes
@@ -1724,7 +1726,7 @@ int launch_scatter(const GatherArgs& a, hipStream_t stream, int K = 1, const Mod
     }
     return PTY_OK;
   }
-  const ScatterPlan plan = modes_plan(a, K);
+  const ScatterPlan plan = stage_plan(a, K);
   const dim3 grid(scatter_blocks(plan), K), blk(256);
   if (plan.rows_per_lane == 1) hipLaunchKernelGGL(k_scatter<1>, grid, blk, 0, stream, a, plan, m);
   else hipLaunchKernelGGL(k_scatter<4>, grid, blk, 0, stream, a, plan, m);
@@ -1815,7 +1817,7 @@ int launch_scatter_probe(const GatherArgs& g, const ProbePartialArgs& pa, hipStr
     }
     return PTY_OK;
   }
-  const ScatterPlan plan = modes_plan(g, K);
+  const ScatterPlan plan = stage_plan(g, K);
   const int ns = scatter_blocks(plan);
   const int rp = probe_pixels_per_lane(pa.S, nchunk), pix_blocks = pa.S * pa.S / (rp * PROBE_PIX);
   const dim3 grid(ns + pix_blocks * nchunk, K), blk(256);
