@@ -1,7 +1,7 @@
 """Batched runs choose the scatter's tile and the probe sums' pixels per lane
 by all problems together, single runs by their own object and batch: results
-stay bitwise those of the single runs on either side of both rules (64 x 4096
-object pixels with at most 25 windows a pixel and round of work groups; 1024
+stay bitwise those of the single runs on either side of both rules (25 windows
+a pixel times the objects' share of 64 x 4096 pixels, squared below one; 1024
 work groups at one pixel per lane), with short last stages and with fixed
 probes between updated ones."""
 
@@ -15,15 +15,15 @@ torch = pytest.importorskip("torch")
 
 # (frame, object, scan, batch, fixed probe) of each problem; stage
 CASES = {
-    # 180,000 pixels, 512 work groups: as the single runs
-    "small-tiles-one-pixel": ([(128, 300, 6, 36, False), (128, 300, 7, 25, False)], 0),
-    # 289,600 pixels, 8.4 windows a pixel, 576 work groups
+    # 54,500 pixels, 34 windows a pixel, 512 work groups
+    "small-tiles-one-pixel": ([(128, 160, 7, 49, False), (128, 170, 8, 64, False)], 0),
+    # 289,600 pixels, 8.9 windows a pixel, 576 work groups
     "wide-tiles-one-pixel": ([(128, 300, 6, 36, False), (128, 300, 7, 49, True),
                               (128, 300, 8, 64, False), (64, 140, 8, 30, False)], 0),
-    # 178,601 pixels, 1,728 work groups
+    # 178,601 pixels, 28 windows a pixel, 1,728 work groups
     "small-tiles-four-pixels": ([(128, 300, 9, 81, False), (128, 261, 11, 121, False),
                                  (64, 64, 12, 144, False), (128, 128, 9, 70, False)], 0),
-    # 310,000 pixels, 18 windows a pixel, 1,152 work groups, stages of 128 with remainders
+    # 310,000 pixels, 17 windows a pixel, 1,152 work groups, stages of 128 with remainders
     "wide-tiles-four-pixels-staged": ([(128, 300, 9, 81, False), (128, 300, 12, 144, False),
                                        (64, 200, 12, 130, False), (128, 300, 9, 81, True)], 128),
 }
