@@ -1919,7 +1919,7 @@ __global__ __launch_bounds__(256) void k_object_expi(const float* __restrict__ p
 int launch_object_gaussian(cf* obj, int Px, int Py, const double* w, int r, int pure, void* tmp,
                            hipStream_t stream) {
   const long long npix = (long long)Px * Py;
-  const dim3 grid(grid_for(npix, 256)), blk(256);
+  const dim3 grid((unsigned)((npix + 255) / 256)), blk(256);  // one pixel a thread
   if (pure) {
     float* ph = (float*)tmp;
     float* ph2 = ph + npix;
@@ -1939,7 +1939,7 @@ int launch_object_gaussian(cf* obj, int Px, int Py, const double* w, int r, int 
 // Px * Py * 4 bytes
 int launch_gaussian_real(float* V, int Px, int Py, const double* w, int r, void* tmp, hipStream_t stream) {
   const long long npix = (long long)Px * Py;
-  const dim3 grid(grid_for(npix, 256)), blk(256);
+  const dim3 grid((unsigned)((npix + 255) / 256)), blk(256);  // one pixel a thread
   float* t = (float*)tmp;
   hipLaunchKernelGGL((k_gaussian_axis<float, 0>), grid, blk, 0, stream, V, t, Px, Py, w, r);
   hipLaunchKernelGGL((k_gaussian_axis<float, 1>), grid, blk, 0, stream, t, V, Px, Py, w, r);
