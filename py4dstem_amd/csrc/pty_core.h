@@ -1858,4 +1858,10 @@ template <class Run> PTY_HD void gather_tile(Run& run, const GatherArgs& a, int 
   });
 }
 
+// Whether a DFT product of M rows over n points runs on 16 x 16 tiles with its
+// roots in LDS: 64 KiB of them, and a row of tiles per y index of the grid
+// (65,536 at most); otherwise 32 x 32 tiles.
+constexpr int DFT_MAX = 8192, GRID_Y_MAX = 65536;
+PTY_HD bool dft_in_lds(int M, int n) { return n <= DFT_MAX && M <= 16 * GRID_Y_MAX; }
+
 }  // namespace pty

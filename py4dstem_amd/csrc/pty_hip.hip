@@ -2030,7 +2030,6 @@ __device__ __forceinline__ cf dft_epilogue(const DftArgs& a, cf v, int x, int y,
 // product, division or trigonometry is left in the loop.  At 284 x 272 pixels
 // a product took 48 us on 32 x 32 tiles with a sincospi per tile element
 // (81 work groups), and takes 8 to 10 us here.
-constexpr int DFT_MAX = 8192;  // roots that fit 64 KiB of LDS
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <bool LEFT> __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
@@ -2110,7 +2109,7 @@ template <bool LEFT> __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
   if (row < a.M && col < a.N) a.Y[(size_t)row * a.N + col] = dft_epilogue(a, partial[0][64 * e + lane], row, col, mean);
 }
 
-// more than DFT_MAX points: roots generated tile by tile
+// beyond dft_in_lds: roots generated tile by tile
 template <bool LEFT>
 __global__ __launch_bounds__(256) void k_dft_any(DftArgs a) {
   __shared__ cf As[DFT_T][DFT_T + 1];
@@ -2274,7 +2273,7 @@ __global__ __launch_bounds__(256) void k_complex_sum_partial(const cf* __restric
 
 template <bool LEFT> void launch_dft(const DftArgs& a, hipStream_t stream) {
   const int n = LEFT ? a.M : a.N;
-  if (n <= DFT_MAX)
+  if (dft_in_lds(a.M, n))
     hipLaunchKernelGGL(k_dft<LEFT>, dim3((a.N + 15) / 16, (a.M + 15) / 16), dim3(256), (size_t)n * sizeof(cf), stream, a);
   else
     hipLaunchKernelGGL(k_dft_any<LEFT>, dim3((a.N + DFT_T - 1) / DFT_T, (a.M + DFT_T - 1) / DFT_T), dim3(256), 0, stream,

@@ -279,6 +279,8 @@ int emu_gather(int S, const float* ps, const float* chi, const float* positions,
   return 0;
 }
 
+int emu_dft_in_lds(int M, int n) { return dft_in_lds(M, n); }
+
 int emu_gather_num_tiles(int Px, int Py) { return gather_num_tiles(Px, Py); }
 
 // the same scatter in stages of `stage` slots with float64 sums carried over
