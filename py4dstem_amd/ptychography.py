@@ -135,10 +135,11 @@ def upload(dev, arrays):
 
 def download(tensors):
     """Host arrays of contiguous device tensors."""
-    out = [None] * len(tensors)
-    small = [i for i, t in enumerate(tensors) if 0 < t.numel() * t.element_size() <= _PACK_BYTES]
+    out, small = [None] * len(tensors), []
     for i, t in enumerate(tensors):
-        if i not in small:
+        if 0 < t.numel() * t.element_size() <= _PACK_BYTES:
+            small.append(i)
+        else:
             out[i] = t.cpu().numpy()
     if small:
         parts = []
