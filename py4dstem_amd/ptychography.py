@@ -98,9 +98,12 @@ def subdivide_into_batches(num_items, max_batch):
 # 23 us down whatever its size below some hundred KiB (a pass over 1,024
 # positions of 64 px in eight iterations, 737 us: three up and a fill, three
 # down; 707 us with one of each, 544 against 592 us over 256 positions of 32 px,
-# 6.18 against 6.62 ms for twelve problems side by side).  Results above _PACK_BYTES go by themselves: there the copy costs
-# more than the call, and the packed copy would need as much memory again.
+# 6.18 against 6.62 ms for twelve problems side by side).  Results above
+# _PACK_BYTES go by themselves: there the copy costs more than the call, and the
+# packed copy would need as much memory again.
 _PACK_BYTES = 1 << 20
+# A result keeps the buffer it came in alive: at most this much of the others'.
+_PACK_TOTAL = 16 << 20
 _ALIGN = 256
 
 
@@ -135,26 +138,35 @@ def upload(dev, arrays):
 
 def download(tensors):
     """Host arrays of contiguous device tensors."""
-    out, small = [None] * len(tensors), []
+    out, small, held = [None] * len(tensors), [], 0
     for i, t in enumerate(tensors):
-        if 0 < t.numel() * t.element_size() <= _PACK_BYTES:
-            small.append(i)
-        else:
+        n = t.numel() * t.element_size()
+        if not 0 < n <= _PACK_BYTES:
             out[i] = t.cpu().numpy()
+            continue
+        if held + n > _PACK_TOTAL:
+            _download_packed(tensors, small, out)
+            small, held = [], 0
+        small.append(i)
+        held += n
     if small:
-        parts = []
-        for i in small:  # each begins at a multiple of eight bytes
-            parts.append(tensors[i].reshape(-1).view(torch.uint8))
-            if parts[-1].numel() % 8:
-                parts.append(parts[-1].new_empty(8 - parts[-1].numel() % 8))
-        host = torch.cat(parts).cpu().numpy()
-        at = 0
-        for i in small:
-            t = tensors[i]
-            n = t.numel() * t.element_size()
-            out[i] = host[at:at + n].view(_NUMPY_DTYPE[t.dtype]).reshape(tuple(t.shape))
-            at += -(-n // 8) * 8
+        _download_packed(tensors, small, out)
     return out
+
+
+def _download_packed(tensors, small, out):
+    parts = []
+    for i in small:  # each begins at a multiple of eight bytes
+        parts.append(tensors[i].reshape(-1).view(torch.uint8))
+        if parts[-1].numel() % 8:
+            parts.append(parts[-1].new_empty(8 - parts[-1].numel() % 8))
+    host = torch.cat(parts).cpu().numpy()
+    at = 0
+    for i in small:
+        t = tensors[i]
+        n = t.numel() * t.element_size()
+        out[i] = host[at:at + n].view(_NUMPY_DTYPE[t.dtype]).reshape(tuple(t.shape))
+        at += -(-n // 8) * 8
 
 
 _NUMPY_DTYPE = {torch.complex64: np.complex64, torch.float32: np.float32, torch.float64: np.float64}

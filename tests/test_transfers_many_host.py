@@ -25,3 +25,19 @@ def test_time_grows_with_the_number_of_results():
 
     best(10)
     assert best(30000) < 30 * best(3000)
+
+
+def test_a_kept_result_holds_a_bounded_buffer():
+    from py4dstem_amd import ptychography as P
+    tensors = [torch.full((200, 300), float(i)) for i in range(150)] + [torch.zeros(0), torch.ones(3)]
+    back = P.download(tensors)
+
+    def held(a):
+        while isinstance(a.base, np.ndarray):
+            a = a.base
+        return a.nbytes
+
+    assert sum(a.nbytes for a in back) > 2 * 16 * 2 ** 20
+    assert max(held(a) for a in back) <= 16 * 2 ** 20 + 8 * len(back)
+    for a, t in zip(back, tensors):
+        np.testing.assert_array_equal(a, t.numpy())
