@@ -9,7 +9,7 @@
 //                    separated by wave barriers, everything else by
 //                    work-group barriers (nine per position).
 //   k_scatter        one work group per object tile: float64 sums of the
-//                    staged patches in batch order (pty_scatter.inc).
+//                    staged patches in batch order (pty_scatter.h).
 //   k_scatter_probe  the scatter and the probe's chunk sums in one launch.
 //   k_update_reduce  normalised object step beside the probe's reduction;
 //   k_probe_apply*   probe step and fft2 of the new probe.
@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "pty_core.h"
+#include "pty_scatter.h"
 #include "../../include/pty_hip.h"
 
 using namespace pty;
@@ -557,7 +558,37 @@ __host__ __device__ inline GatherArgs gather_mode(GatherArgs g, const ModeStride
   return g;
 }
 
-#include "pty_scatter.inc"
+template <int R> struct ScatterGpuRunner {
+  typename Scatter<R>::Regs& r;
+  ScatterSharedView<R> sh;
+  int tid;
+  template <class Fn> __device__ __forceinline__ void phase(Fn fn) { fn(tid, r, sh); }
+  __device__ __forceinline__ void barrier() { __syncthreads(); }
+  __device__ __forceinline__ void ballot() {
+#pragma unroll
+    for (int k = 0; k < Scatter<R>::CAND; ++k) r.mask[k] = __ballot(r.hit[k]);
+  }
+  __device__ __forceinline__ void wave_max() {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) r.max = fmaxf(r.max, __shfl_xor(r.max, off));
+  }
+  template <class Fn> __device__ __forceinline__ int uniform(Fn fn) { return fn(r); }
+};
+
+template <int R>
+__device__ __forceinline__ void scatter_body(const GatherArgs& a, const ScatterPlan& plan, int blk,
+                                             ScatterShared<R>& sh) {
+  typename Scatter<R>::Regs r;
+  ScatterGpuRunner<R> run{r, ScatterSharedView<R>{&sh}, (int)threadIdx.x};
+  scatter_tile<R>(run, a, plan, blk);
+}
+
+template <int R>
+__global__ __launch_bounds__(SCATTER_THREADS) void k_scatter(GatherArgs a, ScatterPlan plan, ModeStride m) {
+  __shared__ ScatterShared<R> sh;
+  if (gridDim.y > 1) a = gather_mode(a, m, blockIdx.y);
+  scatter_body<R>(a, plan, (int)blockIdx.x, sh);
+}
 
 // Correctly rounded float32 square root of x >= 0 (IEEE / NumPy semantics).
 // The hardware estimate r is within one ulp.  The midpoints between r and its

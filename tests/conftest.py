@@ -28,7 +28,8 @@ def emu():
 
     if not os.path.exists(EMU_LIB) or os.path.getmtime(EMU_LIB) < max(
             os.path.getmtime(EMU_SRC),
-            os.path.getmtime(os.path.join(ROOT, "py4dstem_amd", "csrc", "pty_core.h"))):
+            os.path.getmtime(os.path.join(ROOT, "py4dstem_amd", "csrc", "pty_core.h")),
+            os.path.getmtime(os.path.join(ROOT, "py4dstem_amd", "csrc", "pty_scatter.h"))):
         build_emulator()
     lib = ctypes.CDLL(EMU_LIB)
     lib.emu_violations.restype = ctypes.c_long

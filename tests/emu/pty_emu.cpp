@@ -18,6 +18,7 @@ static void note_violation(const char* what) {
 #define PTY_CHECK(cond, what) ((cond) ? (void)0 : note_violation(what))
 
 #include "../../py4dstem_amd/csrc/pty_core.h"
+#include "../../py4dstem_amd/csrc/pty_scatter.h"
 
 using namespace pty;
 
@@ -162,6 +163,100 @@ struct GatherEmu {
   void barrier() { scan0.clear(); scan1.clear(); list.clear(); red.clear(); }
 };
 
+template <int R> struct ScatterEmu {
+  using K = Scatter<R>;
+  int cur = -1;
+  TrackedArr<ScatterHit> list{SCATTER_SEG};
+  TrackedArr<float> prod{2 * 3 * K::CHUNK * K::TP};
+  TrackedArr<int> count{4};
+  TrackedArr<float> red{4};
+  std::vector<typename K::Regs> regs = std::vector<typename K::Regs>(SCATTER_THREADS);
+  struct View {
+    ScatterEmu* e;
+    LdsArrCheck<ScatterHit> list() const { return e->list.view(&e->cur); }
+    LdsArrCheck<float> prod() const { return e->prod.view(&e->cur); }
+    LdsArrCheck<int> count() const { return e->count.view(&e->cur); }
+    LdsArrCheck<float> red() const { return e->red.view(&e->cur); }
+  };
+  template <class Fn> void phase(Fn fn) {
+    for (int t = 0; t < SCATTER_THREADS; ++t) {
+      cur = t;
+      fn(t, regs[t], View{this});
+    }
+    cur = -1;
+  }
+  void barrier() { list.clear(); prod.clear(); count.clear(); red.clear(); }
+  void ballot() {
+    for (int w = 0; w < SCATTER_THREADS; w += WAVE)
+      for (int k = 0; k < K::CAND; ++k) {
+        unsigned long long m = 0;
+        for (int t = 0; t < WAVE; ++t) m |= (unsigned long long)regs[w + t].hit[k] << t;
+        for (int t = 0; t < WAVE; ++t) regs[w + t].mask[k] = m;
+      }
+  }
+  void wave_max() {
+    for (int w = 0; w < SCATTER_THREADS; w += WAVE) {
+      float m = 0.f;
+      for (int t = 0; t < WAVE; ++t) m = fmaxf(m, regs[w + t].max);
+      for (int t = 0; t < WAVE; ++t) regs[w + t].max = m;
+    }
+  }
+  template <class Fn> int uniform(Fn fn) {
+    for (const auto& r : regs)
+      if (fn(r) != fn(regs[0])) note_violation("value not uniform over the work group");
+    return fn(regs[0]);
+  }
+};
+
+// the frames of one launch, tiles of R rows per lane
+template <int R> static void run_scatter(const GatherArgs& a) {
+  ScatterPlan plan = scatter_plan(a.Px, a.Py, R);
+  if (R == 4) plan.num_tiles = scatter_plan(a.Px, a.Py, 1).num_tiles;  // the rest cleared
+  for (int blk = 0; blk < scatter_blocks(plan); ++blk) {
+    ScatterEmu<R> run;
+    scatter_tile<R>(run, a, plan, blk);
+  }
+}
+
+static void run_gather(const GatherArgs& a) {
+  for (int tile = 0; tile < gather_num_tiles(a.Px, a.Py); ++tile) {
+    GatherEmu run;
+    gather_tile(run, a, tile);
+  }
+}
+
+// `launches` (one per stage, in order) through `run`, with outputs and running
+// sums of its own; a violation where they differ from `want` in any bit
+template <class Run>
+static void same_outputs(const std::vector<GatherArgs>& launches, const GatherArgs& want, Run run, const char* what) {
+  const size_t n = (size_t)want.Px * want.Py, tiles = scatter_plan(want.Px, want.Py, 1).num_tiles;
+  std::vector<cf> grad(n);
+  std::vector<float> spsum(n), tilemax(tiles, -1.f);
+  std::vector<double> sums(3 * n);
+  for (GatherArgs a : launches) {
+    a.grad = grad.data(); a.spsum = spsum.data(); a.tilemax = tilemax.data();
+    if (a.run) a.run = sums.data();
+    run(a);
+  }
+  float m = 0.f, ms = 0.f;
+  for (float v : tilemax) {
+    if (v < 0.f) note_violation("tile maximum not written");
+    m = fmaxf(m, v);
+  }
+  for (float v : spsum) ms = fmaxf(ms, v);
+  if (m != ms) note_violation("tile maxima differ from the sums");
+  if (std::memcmp(grad.data(), want.grad, n * sizeof(cf)) || std::memcmp(spsum.data(), want.spsum, n * sizeof(float)))
+    note_violation(what);
+}
+
+// through all three kernels' phases; the caller's buffers get the one that
+// serves frames of any size
+static void scatter_all(const std::vector<GatherArgs>& launches) {
+  for (const GatherArgs& a : launches) run_gather(a);
+  same_outputs(launches, launches.back(), run_scatter<1>, "scatter of 64-pixel tiles differs");
+  same_outputs(launches, launches.back(), run_scatter<4>, "scatter of 256-pixel tiles differs");
+}
+
 template <int S> static void run_fused(const FusedArgs& a) {
   EmuRunner<S> run(&a);
   for (int b = a.b0; b < a.B; ++b) fused_position<S>(run, a, b);
@@ -272,10 +367,7 @@ int emu_gather(int S, const float* ps, const float* chi, const float* positions,
   a.N = N; a.B = B; a.S = S; a.Px = Px; a.Py = Py;
   a.tiles_y = gather_tiles_y(Py);
   a.grad = (cf*)grad; a.spsum = spsum; a.tilemax = tilemax;
-  for (int tile = 0; tile < gather_num_tiles(Px, Py); ++tile) {
-    GatherEmu run;
-    gather_tile(run, a, tile);
-  }
+  scatter_all({a});
   return 0;
 }
 
@@ -287,6 +379,7 @@ int emu_gather_num_tiles(int Px, int Py) { return gather_num_tiles(Px, Py); }
 int emu_gather_staged(int S, const float* ps, const float* chi, const float* positions, int N,
                       const int* order, int B, int stage, int Px, int Py, float* grad, float* spsum,
                       float* tilemax, double* runbuf) {
+  std::vector<GatherArgs> launches;
   for (int s0 = 0; s0 < B; s0 += stage) {
     const int ns = (B - s0) < stage ? (B - s0) : stage;
     GatherArgs a{};
@@ -295,11 +388,9 @@ int emu_gather_staged(int S, const float* ps, const float* chi, const float* pos
     a.N = N; a.B = ns; a.S = S; a.Px = Px; a.Py = Py; a.tiles_y = gather_tiles_y(Py);
     a.grad = (cf*)grad; a.spsum = spsum; a.tilemax = tilemax;
     a.run = runbuf; a.run_first = s0 == 0; a.run_last = s0 + ns == B;
-    for (int tile = 0; tile < gather_num_tiles(Px, Py); ++tile) {
-      GatherEmu run;
-      gather_tile(run, a, tile);
-    }
+    launches.push_back(a);
   }
+  scatter_all(launches);
   return 0;
 }
 
