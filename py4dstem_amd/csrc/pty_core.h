@@ -846,7 +846,7 @@ template <int S> struct Fused {
   // overlap psi = P * O_patch, previous exit wave e (psi on the first
   // iteration), c psi + y e into the forward column pass, and the partial
   // new exit wave w = x e + a psi (the reference's left-to-right float32
-  // evaluation order), which stays in registers: at 128 px that spills 8 of
+  // evaluation order), which stays in registers: at 128 px that spills 11 of
   // them, and parking it in the exit wave's frame instead moved 256 KB more a
   // position (2,968 positions: 581 against 428 us a launch)
   template <class L> static PTY_HD void p_proj_colA(int tid, const FusedArgs& a, int b, Regs& r,
@@ -1541,7 +1541,9 @@ PTY_HD void position_correction_position(Run& run, const PosArgs& a, int b) {
 }
 
 // ---------------------------------------------------------------------------
-// Deterministic scatter-add by object pixel ("sort by pixel").  One work group
+// Deterministic scatter-add by object pixel ("sort by pixel"), with element
+// offsets for frames of any size: launches of more than 2 GiB of frames (the
+// others take the tiles of pty_scatter.h, with the same sums).  One work group
 // owns a TR x TC object tile, GT_RPT pixels of one column per thread (the
 // column test of a hit is shared by them; the 64 lanes of a wave read 512
 // contiguous bytes of a patch row).  For each segment of the

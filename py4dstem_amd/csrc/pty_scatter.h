@@ -47,9 +47,9 @@ template <int R> struct ScatterTile {
 constexpr int SCATTER_SEG = 1024;  // batch slots per hit list
 constexpr int SCATTER_THREADS = 256;
 
-// Up to this many object pixels the 64-pixel tiles are used: 4096 work
-// groups, about four rounds of the 1024 that fit the chip (LDS).  Measured
-// with 128 px frames: 284x272 pixels 45 us against 115 us with 256-pixel
+// Beyond this many object pixels the 256-pixel tiles are used: 4096 work
+// groups of 64 pixels are about four rounds of the 1024 that fit the chip
+// (LDS).  Measured where hundreds of windows overlap, with 128 px frames: 284x272 pixels 45 us against 115 us with 256-pixel
 // tiles, 440x416 (256 px frames) 32 against 42, 720^2 74 against 56.
 constexpr long long SCATTER_SMALL_PIXELS = 64 * 4096;
 
